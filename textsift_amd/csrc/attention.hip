@@ -623,16 +623,33 @@ __global__ __launch_bounds__(64 * NW) void k_banded_attention_hw(AttnArgs a) {
   }
 }
 
+// Workgroups per KV head: its G query heads are split evenly over them (each
+// stages the K/V rows for its own heads). The launch takes rounds of
+// `resident` workgroups at a time, each as long as its largest share of heads
+// plus the staging, which costs about one head (34 us for 7 heads, 23 us for
+// 4): the split with the least rounds x (heads + 1), the coarsest on a tie.
+// (The fewest workgroups that give every CU one, the earlier rule, took two
+// rounds of 4 heads at 12 x 1000 tokens, where one round of 7 fits: 9 us more.)
+int attn_head_groups(long wgs, int G, long resident) {
+  int best = 1;
+  long cost = -1;
+  for (int g = 1; g <= G; ++g) {
+    const long c = ((wgs * g + resident - 1) / resident) * ((G + g - 1) / g + 1);
+    if (cost < 0 || c < cost) {
+      best = g;
+      cost = c;
+    }
+  }
+  return best;
+}
+
 template <typename Kern>
 void launch_kernel(pfhip_backend* b, const AttnArgs& a, Kern* kern, size_t lds, int qb, int nt) {
   allow_lds(reinterpret_cast<const void*>(kern), lds);
-  // few workgroups (short inputs): the query heads of a KV head are split
-  // over several workgroups (the fewest that give every CU one), so they run
-  // in parallel; each still stages its K/V rows once for all its heads
   AttnArgs g = a;
   const long wgs = (long)((a.T + qb - 1) / qb) * a.Hkv * a.B;
-  const int G = a.Hq / a.Hkv;
-  g.head_groups = (int)std::min<long>(G, (b->num_cus + wgs - 1) / wgs);
+  // resident workgroups: the 8-wave tiles hold 2 waves per SIMD (registers), the 4-wave ones 3
+  g.head_groups = attn_head_groups(wgs, a.Hq / a.Hkv, (long)b->num_cus * (nt > 256 ? 1 : 3));
   dim3 grid((a.T + qb - 1) / qb, a.Hkv * g.head_groups, a.B);
   ProfScope ps(b, "banded_attention");
   hipLaunchKernelGGL(kern, grid, dim3(nt), lds, b->stream, g);
