@@ -65,3 +65,19 @@ def test_attention_key_mask(be, T, W, hw_exp):
     err, same = rel_err_norm(f16(out), f16(ref)), np.mean(out == ref)
     print(f"attention mask T={T} W={W} hw_exp={hw_exp}: rel-err {err:.3e}, identical {same:.4f}, {zero.sum()} empty rows")
     assert err < (5e-4 if hw_exp else 2e-3) and same > (0.5 if hw_exp else 0.97)
+
+
+# ---------------------------------------------------------------- conversions
+
+@pytest.mark.parametrize("scale", [1.0, 2.0 ** -14, 2.0 ** -24])
+def test_fp16_narrowing_below_normal(be, scale):
+    """fp16 narrowing with round-half-up below 2^-14: values around every
+    subnormal's halfway points, signed zeros, the normal boundary, infinities and NaN, bit for bit."""
+    n = np.arange(0, 1026, dtype=np.float64)
+    v = np.concatenate([(n + d) * 2.0 ** -24 for d in (-0.5, -0.4999999, 0.0, 0.4999999, 0.5, 0.5000001)])
+    v = np.concatenate([v, -v, [0.0, -0.0, 2.0 ** -26, 65504.0, 65519.0, 65520.0, np.inf, -np.inf, np.nan, 1e-40]])
+    s = np.resize((v.astype(np.float32) / np.float32(scale)).astype(np.float32), 12800)
+    got = run(be, "cast_f32_to_fp16_scaled", [s], s.size * 2,
+              u32s(s.size, 0, 0, 0) + struct.pack("<f", scale) + u32s(0, 0, 0)).view(np.uint16)
+    ref = oracle.f32_to_fp16(s * np.float32(scale))
+    assert np.array_equal(got, np.asarray(ref, np.uint16))

@@ -39,23 +39,19 @@ __device__ __forceinline__ float f32_fence(float f) {
   return f;
 }
 
+// Branch-free, so a wave with one subnormal result does not run a second
+// path: below 2^-14 the result's bits are |f| 2^24 (exact) rounded half up
+// (1024 is the smallest normal; below 2^-25 it gives 0 by itself).
 __device__ __forceinline__ uint16_t wasm_f2h(float f) {
   f = f32_fence(f);
   const float a = fabsf(f);
-  if (a >= 6.103515625e-05f || !(a == a)) {
-    _Float16 h = (_Float16)f;
-    uint16_t bits = __builtin_bit_cast(uint16_t, h);
-    if (!(a == a)) bits = (uint16_t)((bits & 0x8000u) | 0x7e00u);  // NaN: quiet bit (math.zig:59)
-    return bits;
-  }
-  uint32_t u = __float_as_uint(f);
-  uint32_t sign = (u >> 16) & 0x8000u;
-  uint32_t exp32 = (u >> 23) & 0xffu;
-  int32_t e16 = (int32_t)exp32 - 127 + 15;
-  if (e16 < -10) return (uint16_t)sign;
-  uint32_t shift = (uint32_t)(14 - e16);
-  uint32_t mant24 = (u & 0x7fffffu) | 0x800000u;
-  return (uint16_t)(sign | ((mant24 + (1u << (shift - 1))) >> shift));
+  const uint32_t hw = __builtin_bit_cast(uint16_t, (_Float16)f);
+  const float v = fminf(a * 16777216.0f, 1024.0f), n = floorf(v);
+  const uint32_t sub = (uint32_t)n + (v - n >= 0.5f ? 1u : 0u);  // (unused from 2^-14 on)
+  const uint32_t sign = (__float_as_uint(f) >> 16) & 0x8000u;
+  uint32_t bits = a >= 6.103515625e-05f ? hw : (sign | sub);
+  if (!(a == a)) bits = sign | 0x7e00u;  // NaN: quiet bit (math.zig:59)
+  return (uint16_t)bits;
 }
 
 // True when the fp16 rounding of f involves none of the cases in which the
@@ -94,6 +90,16 @@ __device__ __forceinline__ void copy16_to_lds(const void* src, lds_ptr_t dst) {
 #if defined(__HIP_DEVICE_COMPILE__)
   __builtin_amdgcn_global_load_lds(src, dst, 16, 0, 0);
 #endif
+}
+
+// copy16_to_lds issued as inline assembly: the compiler then does not know
+// that it writes LDS and does not make every workgroup barrier wait for all
+// such copies in flight (vmcnt(0)); the kernel waits for the ones it needs
+// itself. Clobbers M0, which nothing else in the kernel uses. An LDS DMA
+// reads M0 one wait state after the write at the earliest (the s_nop).
+__device__ __forceinline__ void copy16_to_lds_async(const void* src, uint32_t lds_byte) {
+  asm volatile("s_mov_b32 m0, %1\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %0, off" : : "v"(src), "s"(lds_byte)
+               : "memory", "m0");
 }
 
 // True when wasm_h2f of each of the four fp16 values packed in w is the

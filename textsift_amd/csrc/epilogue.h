@@ -43,6 +43,33 @@ __device__ __forceinline__ void rope_pair_exact(uint16_t& ha, uint16_t& hb, floa
   hb = wasm_f2h(bc + as_);
 }
 
+// wasm_h2f(wasm_f2h(x)) for |x| <= 65504, branch-free: a subnormal result n
+// 2^-24 (n = |x| 2^24 rounded half up) widens to 2^-15 + n 2^-25, zero to zero.
+__device__ __forceinline__ float wasm_round16(float x) {
+  x = f32_fence(x);
+  const float a = fabsf(x), v = fminf(a * 16777216.0f, 1024.0f);
+  float n = floorf(v);
+  n = v - n >= 0.5f ? n + 1.0f : n;
+  const float sub = n == 0.0f ? 0.0f : fmaf(n, 2.98023223876953125e-08f, 3.0517578125e-05f);
+  return copysignf(a >= 6.103515625e-05f ? (float)(_Float16)a : sub, x);
+}
+
+// The rotation of two pairs when every value lies within +-65504: what
+// rope_f16x4_exact gives, without its software conversions. The tables'
+// low-frequency sines put subnormal products in nearly every wave, so this
+// path is taken more often than not.
+__device__ __noinline__ u2_t rope_f16x4_small(f4_t v, f2_t cs, f2_t sn) {
+  uint16_t hb[4];
+#pragma unroll
+  for (int h = 0; h < 2; ++h) {
+    const float x0 = v[2 * h], x1 = v[2 * h + 1], c = cs[h], s = sn[h];
+    const float a = wasm_round16(x0), b = wasm_round16(x1);
+    hb[2 * h] = wasm_f2h(wasm_round16(a * c) - wasm_round16(b * s));
+    hb[2 * h + 1] = wasm_f2h(wasm_round16(b * c) + wasm_round16(a * s));
+  }
+  return pack4(hb);
+}
+
 __device__ __noinline__ u2_t rope_f16x4_exact(f4_t v, f2_t cs, f2_t sn) {
   uint16_t hb[4];
 #pragma unroll
@@ -108,8 +135,10 @@ __device__ __forceinline__ u2_t rope_f16x4(const float v[4], f2_t cs, f2_t sn) {
     hb[2 * h] = hw_f2h(r0);
     hb[2 * h + 1] = hw_f2h(r1);
   }
-  // NaN anywhere makes both comparisons false
-  if (!(lo >= 6.103515625e-05f && hi <= 65504.0f)) return rope_f16x4_exact(f4_t{v[0], v[1], v[2], v[3]}, cs, sn);
+  // NaN anywhere makes the comparison false (a NaN product or sum comes from a NaN or infinite v; fmaxf skips NaN)
+  if (!(hi <= 65504.0f) || v[0] != v[0] || v[1] != v[1] || v[2] != v[2] || v[3] != v[3])
+    return rope_f16x4_exact(f4_t{v[0], v[1], v[2], v[3]}, cs, sn);
+  if (!(lo >= 6.103515625e-05f)) return rope_f16x4_small(f4_t{v[0], v[1], v[2], v[3]}, cs, sn);
   return pack4(hb);
 }
 
