@@ -67,7 +67,57 @@ def test_attention_key_mask(be, T, W, hw_exp):
     assert err < (5e-4 if hw_exp else 2e-3) and same > (0.5 if hw_exp else 0.97)
 
 
-# ---------------------------------------------------------------- conversions
+# ---------------------------------------------------------------- int4 GEMM, split numerics
+
+@pytest.mark.parametrize("x_f32", [True, False], ids=["f32", "fp16"])
+@pytest.mark.parametrize("T,N,K,zp", [(1, 33, 128, 8), (31, 64, 640, None), (33, 96, 896, None), (70, 130, 384, 8),
+                                      (65, 640, 1024, None), (4111, 72, 640, 8)])
+def test_matmul_int4_chunked(be, T, N, K, zp, x_f32):
+    """The K % 128 == 0 kernel: partial token and column tiles, odd, even and
+    compile-time chunk counts, zero-points of every block, both activation
+    forms and the 64-token tile. The f32 output against the oracle: both sum the
+    same per-block products in f32, so the difference is a few f32 ulps of the
+    largest partial sum (K / 32 blocks: 2^-23 sqrt(K / 32) relative, times 4), plus 2^-22 for the hi/lo split."""
+    w = synth.qweight(1300 + K, N, K, zp=zp)
+    x = synth.normal(1301 + T, T * K).astype(np.float32).reshape(T, K)
+    xin = x if x_f32 else synth.to_fp16_bits(x).reshape(T, K)
+    name = "matmul_int4_f32_f32" if x_f32 else "matmul_int4_fp16_f32"
+    got = run(be, name, [xin, w["int4"], w["scales"], w["zp"], w["bias"]], T * N * 4, u32s(T, N, K, 0))
+    ref = oracle.matmul(xin, w["int4"], w["scales"], w["zp"], w["bias"], N, K, x_f32=x_f32, out_f32=True)
+    err = rel_err_norm(got.view(np.float32), ref.ravel())
+    print(f"matmul T={T} N={N} K={K} zp={zp} x_f32={x_f32}: rel-err {err:.2e}")
+    assert err < 4 * 2.0 ** -23 * np.sqrt(K / 32) + 2.0 ** -22
+
+
+@pytest.mark.parametrize("T", [100, 1025, 2049])
+def test_moe_layer_split_expert_tiles(be, T):
+    """The split MoE layer on the 16-, 32- and 64-row expert tiles (3, 32 and
+    64 rows per expert on average) with partial tiles, against the oracle fed the
+    GPU's routing: 32-bit sums rounded once to fp16 (2^-11)."""
+    from textsift_amd.config import PF_CONFIG as cfg
+    D, E, K, F = cfg.hidden_size, 128, 4, cfg.intermediate_size
+    x = synth.normal(1400 + T, T * D).astype(np.float32)
+    r = synth.qweight(1401, E, D)
+    gu, dn = synth.qweight(1402, 2 * F, D, lead=(E,)), synth.qweight(1403, D, F, lead=(E,))
+    bufs = [be.buffer(np.ascontiguousarray(a)) for a in
+            [x] + [r[k] for k in ("int4", "scales", "zp", "bias")] +
+            [q[k] for q in (gu, dn) for k in ("int4", "scales", "zp", "bias")]]
+    outs = [be.buffer(nbytes=n) for n in (T * D * 2, T * K * 4, T * K * 4)]
+    be.dispatch("moe_ffn", bufs + outs, u32s(T, D, E, K, F, 1, 1, 0))
+    y = outs[0].read(np.uint16).reshape(T, D)
+    ridx, rwt = outs[1].read(np.int32).reshape(T, K), outs[2].read(np.float32).reshape(T, K)
+    for b in bufs + outs:
+        b.release()
+    w = {f"layers.0.experts.{n}.{k}": v for n, q in (("gate_up", gu), ("down", dn)) for k, v in q.items()}
+    for nm in ("attn.q_proj", "attn.k_proj", "attn.v_proj", "attn.o_proj", "router"):
+        w.update({f"layers.0.{nm}.{k}": v for k, v in synth.qweight(9, 64, 64).items()})
+    w["layers.0.input_layernorm"] = w["layers.0.post_attention_layernorm"] = np.zeros(D, np.uint16)
+    w["layers.0.attn.sinks"] = np.zeros(cfg.num_heads, np.float32)
+    ref = oracle.expert_dispatch(cfg, w, 0, x.reshape(T, D), ridx, rwt * np.float32(0.25), n_slices=8)
+    err = rel_err_norm(f16(y), f16(ref))
+    print(f"split MoE T={T}: rel-err {err:.2e}")
+    assert err < 2.0 ** -11
+
 
 @pytest.mark.parametrize("scale", [1.0, 2.0 ** -14, 2.0 ** -24])
 def test_fp16_narrowing_below_normal(be, scale):

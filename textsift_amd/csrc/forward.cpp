@@ -38,6 +38,8 @@ namespace pf {
 // 896) below 32; fragments per wave 4, 5 and 1 respectively.
 ExpertTile expert_tile(int M, int topk, int experts, bool fp16, int D, int F) {
   const int per_expert = (int)((long)M * topk / experts);
+  // split numerics, K % 128 == 0: gemm_int4's tiles of 16, 32 and 64 rows (measured there)
+  if (!fp16 && D % 128 == 0 && F % 128 == 0) return {per_expert < 32 ? 16 : per_expert < 64 ? 32 : 64, 1};
   if (per_expert >= 256) return {128, 4};
   const auto small_k = [](int k) { return k == 640 || k == 896; };
   if (fp16 && small_k(D) && small_k(F) && per_expert < 32) return {16, 1};

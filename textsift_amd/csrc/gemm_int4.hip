@@ -30,6 +30,7 @@
 #include "common.h"
 #include "epilogue.h"
 #include "pfhip_internal.h"
+#include <type_traits>
 
 namespace pf {
 
@@ -277,6 +278,390 @@ void launch(pfhip_backend* b, const GemmArgs& a, const char* name) {
   PF_HIP(hipGetLastError());
 }
 
+// ---------------------------------------------------------------- K a multiple of 128
+//
+// The same product, scaled per block in the same order (bit-identical results), for K % 128 == 0, with the
+// memory side rebuilt: the kernel above stages 64 K values per two barriers
+// through registers, dequantises into LDS and has few workgroups.
+//  * Weights are not staged: each of the 4 waves owns WF x 16 weight rows.
+//    Lane (l16, lg) reads block lg of the chunk of row l16 as 16 bytes; a 4 x 4
+//    transpose over the lane groups (two permlane swaps per pair of dwords)
+//    leaves it dword lg of each block, its A fragment of that block's MFMA. A
+//    wave's weights are dequantised once for all BT tokens.
+//  * Activations go HBM -> LDS with global_load_lds (both planes), 128 K
+//    values at a time, double buffered, in 256-byte rows whose 16-byte units
+//    are XOR-swizzled by (row & 15): conflict-free fragment reads, one
+//    barrier per 4 quant blocks.
+//  * The lane's accumulator rows are 4 lg .. + 3 of a fragment, so the f32
+//    scales of the chunk are kept in LDS as [block][row] and read as one
+//    16-byte vector per fragment and block; each thread converts WF of them per chunk.
+// 2048 x 1152 x 640 with the RoPE epilogue: 51.1 us in the kernel above, 21.7
+// here; the 2048-token layer's gate_up and down 85 / 46 -> 66 / 33 us. Of that
+// the 16-byte weight loads and their transpose (instead of four 4-byte loads) are
+// a fifth, and the RoPE epilogue's branch-free subnormal path 4 us.
+// Bound: per 16 x 16 x 32 block two MFMAs (32 cycles) and 4 fmaf (16), plus
+// the dequantisation (17 VALU, 68 cycles) per fragment and BT tokens.
+constexpr int KC = 128;  // K per chunk
+
+//  * CT > 0 (K / 128 at compile time): weights are loaded two chunks ahead
+//    and the barrier waits only for the activations, which are one ahead
+//    (the L2 serves them; the weights come from HBM).
+template <int WF, int BT, bool SPLIT, Epi EPI, bool GROUPED, int CT>
+__global__ __launch_bounds__(256, 2) void k_gemm_int4_k128(GemmArgs p) {
+  constexpr int NPL = SPLIT ? 2 : 1;
+  constexpr int NW = 4, BNW = NW * WF * 16;  // weight rows per workgroup
+  constexpr int TJ = BT / 16;
+  constexpr int PLANE = BT * KC;             // halves per plane per buffer
+  constexpr int XI = BT / (4 * NW);          // 4-row copies per wave and plane
+  static_assert(BT % (4 * NW) == 0, "whole 4-row copies per wave");
+  extern __shared__ __attribute__((aligned(16))) _Float16 xs[];  // [2][NPL][BT][KC], then f32 scales [2][4][BNW]
+  float* sl = reinterpret_cast<float*>(xs + 2 * NPL * PLANE);
+
+  const int tid = threadIdx.x, lane = tid & 63;
+  const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const int l16 = lane & 15, lg = lane >> 4;
+  const int n_tiles = (p.N + BNW - 1) / BNW;
+  int active = (int)gridDim.x;
+  if constexpr (GROUPED) {
+    active = min(active, *p.num_tiles * n_tiles);
+    if ((int)blockIdx.x >= active) return;
+  }
+  const int bid = xcd_remap(blockIdx.x, active);
+  const int nt = bid % n_tiles, tt = bid / n_tiles;
+  int expert = 0, row0, rows;
+  if constexpr (GROUPED) {
+    const int4 ti = reinterpret_cast<const int4*>(p.tiles)[tt];
+    expert = ti.x;
+    row0 = ti.y;
+    rows = ti.z;
+  } else {
+    row0 = tt * BT;
+    rows = min(BT, p.M - row0);
+  }
+  const int n0 = nt * BNW, K = p.K, C = K / KC, nb = K >> 5;
+
+  // Weights, zero-points and scales by buffer loads: one descriptor each in
+  // scalar registers, 32-bit byte offsets per lane, the chunk in the scalar
+  // offset (64-bit addresses per load spilled). Rows past N read row N - 1
+  // (never stored). The host checks that one matrix stays below 2^31 bytes.
+  const __amdgpu_buffer_rsrc_t wrs = __builtin_amdgcn_make_buffer_rsrc(
+      const_cast<uint8_t*>(p.w + (size_t)expert * p.w_gs), 0, p.N * (K >> 1), 0x00020000);
+  const __amdgpu_buffer_rsrc_t srs = __builtin_amdgcn_make_buffer_rsrc(
+      const_cast<uint16_t*>(p.ws + (size_t)expert * p.ws_gs), 0, p.N * nb * 2, 0x00020000);
+  const __amdgpu_buffer_rsrc_t zrs = __builtin_amdgcn_make_buffer_rsrc(
+      const_cast<uint8_t*>(p.wz + (size_t)expert * p.wz_gs), 0, p.wz ? p.N * (nb >> 1) : 0, 0x00020000);
+  uint32_t woff[WF], zoff[WF];  // (a chunk's 4 zero-point nibbles are 2 bytes of a row of nb / 2)
+#pragma unroll
+  for (int f = 0; f < WF; ++f) {
+    const int n = min(n0 + (wave * WF + f) * 16 + l16, p.N - 1);
+    woff[f] = (uint32_t)n * (uint32_t)(K >> 1) + lg * 16;
+    zoff[f] = (uint32_t)n * (uint32_t)(nb >> 1);
+  }
+  // scales: thread tid converts WF consecutive blocks of row tid WF / 4
+  const int srow = tid * WF / 4, sblk = tid * WF % 4;
+  const uint32_t soff = ((uint32_t)min(n0 + srow, p.N - 1) * (uint32_t)nb + sblk) * 2u;
+  const uint16_t* __restrict__ xsrc[NPL];
+  xsrc[0] = static_cast<const uint16_t*>(p.x);
+  if constexpr (SPLIT) xsrc[1] = p.x_lo;
+  int xoff[XI];  // rows past the tile read its last row (never stored)
+#pragma unroll
+  for (int m = 0; m < XI; ++m) {
+    const int r = (m * NW + wave) * 4 + lg;
+    const int lr = row0 + min(r, rows - 1);
+    const int g = p.row_map ? p.row_map[lr] : lr;
+    xoff[m] = g * p.ldx + ((l16 ^ (r & 15)) << 3);
+  }
+
+  struct Wts {
+    u4_t q[WF];
+    uint32_t z[WF];
+    uint32_t s;  // WF fp16 scales
+  };
+  // vector memory instructions of one chunk's weights
+  constexpr int VM_W = 2 * WF + 1;
+  const uint32_t lds0 = (uint32_t)(uintptr_t)(lds_ptr_t)xs;
+  auto load_x = [&](int c, int buf) {
+#pragma unroll
+    for (int pl = 0; pl < NPL; ++pl)
+#pragma unroll
+      for (int m = 0; m < XI; ++m)
+        copy16_to_lds_async(reinterpret_cast<const char*>(xsrc[pl]) + (uint32_t)(xoff[m] + c * KC) * 2u,
+                            __builtin_amdgcn_readfirstlane(
+                                lds0 + (uint32_t)((buf * NPL + pl) * PLANE + (m * NW + wave) * 512) * 2));
+  };
+  auto load_w = [&](int c, Wts& w) {
+#pragma unroll
+    for (int f = 0; f < WF; ++f) {
+      w.q[f] = __builtin_amdgcn_raw_buffer_load_b128(wrs, woff[f], c * 64, 0);
+      w.z[f] = __builtin_amdgcn_raw_buffer_load_b16(zrs, zoff[f], c * 2, 0);  // (0 without zero-points: out of range)
+    }
+    if constexpr (WF == 2) w.s = __builtin_amdgcn_raw_buffer_load_b32(srs, soff, c * 8, 0);
+    else w.s = __builtin_amdgcn_raw_buffer_load_b16(srs, soff, c * 8, 0);
+  };
+
+  // the bias of the lane's 4 columns of each fragment, loaded here so the
+  // epilogue does not wait for it (columns past N: unused values)
+  const uint16_t* __restrict__ BIAS = p.bias ? p.bias + (size_t)expert * p.bias_gs : nullptr;
+  int ncol[WF];
+  uint16_t braw[WF][4];
+#pragma unroll
+  for (int f = 0; f < WF; ++f) {
+    ncol[f] = n0 + (wave * WF + f) * 16 + 4 * lg;
+#pragma unroll
+    for (int r = 0; r < 4; ++r) braw[f][r] = BIAS ? BIAS[min(ncol[f] + r, p.N - 1)] : (uint16_t)0;
+  }
+
+  f4_t acc[WF][TJ];
+#pragma unroll
+  for (int f = 0; f < WF; ++f)
+#pragma unroll
+    for (int j = 0; j < TJ; ++j) acc[f][j] = f4_t{0.f, 0.f, 0.f, 0.f};
+
+  // One chunk = 4 blocks, software-pipelined: block j's MFMAs (hi for every
+  // fragment pair, then lo onto them: independent chains) are issued with
+  // block j + 1's fragment reads in flight, block j + 1's dequantisation and
+  // block j - 1's scaling fmaf between them.
+  // Chunk c: its weights' scales to LDS, the workgroup barrier (after it every
+  // wave is done with the other activation buffer), the next loads, the MFMAs.
+  // ahead: vector memory instructions issued after chunk c's activation copies.
+  auto step = [&](int c, int buf, Wts& w, auto ahead, auto next) {
+    constexpr int A = decltype(ahead)::value;
+    static_assert(A < 64, "vmcnt is 6 bits");
+    __builtin_amdgcn_s_waitcnt((A & 15) | (7 << 4) | (15 << 8) | ((A >> 4) << 14));
+#pragma unroll
+    for (int f = 0; f < WF; ++f) {
+      // (landed: no further wait for them once newer loads are in flight)
+      asm volatile("" : "+v"(w.q[f]), "+v"(w.z[f]));
+      sl[(buf * 4 + sblk + f) * BNW + srow] = wasm_h2f((uint16_t)(w.s >> (16 * f)));
+    }
+    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "workgroup", "local");
+    __builtin_amdgcn_s_barrier();
+    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "workgroup", "local");
+    next();
+    uint32_t wq[WF][4];  // block j's dword of this lane
+#pragma unroll
+    for (int f = 0; f < WF; ++f) {
+      const uint32_t q0 = w.q[f][0], q1 = w.q[f][1], q2 = w.q[f][2], q3 = w.q[f][3];
+      const auto a = __builtin_amdgcn_permlane16_swap(q0, q1, false, false);
+      const auto b = __builtin_amdgcn_permlane16_swap(q2, q3, false, false);
+      const auto e = __builtin_amdgcn_permlane32_swap(a[0], b[0], false, false);
+      const auto o = __builtin_amdgcn_permlane32_swap(a[1], b[1], false, false);
+      wq[f][0] = e[0];
+      wq[f][1] = o[0];
+      wq[f][2] = e[1];
+      wq[f][3] = o[1];
+    }
+    const _Float16* xb = xs + buf * NPL * PLANE;
+    h8_t xf[2][NPL][TJ], wd[2][WF];
+    f4_t sc[2][WF], d[2][WF][TJ];
+    auto read = [&](int j) {
+      const int unit = ((4 * j + lg) ^ l16) << 3;
+#pragma unroll
+      for (int t = 0; t < TJ; ++t)
+#pragma unroll
+        for (int pl = 0; pl < NPL; ++pl)
+          xf[j & 1][pl][t] = *reinterpret_cast<const h8_t*>(xb + pl * PLANE + (16 * t + l16) * KC + unit);
+#pragma unroll
+      for (int f = 0; f < WF; ++f)
+        sc[j & 1][f] = *reinterpret_cast<const f4_t*>(&sl[(buf * 4 + j) * BNW + (wave * WF + f) * 16 + 4 * lg]);
+    };
+    auto dequant = [&](int j) {
+#pragma unroll
+      for (int f = 0; f < WF; ++f) {
+        const uint32_t hz = 0x6400u + ((w.z[f] >> (4 * j)) & 0xFu);  // fp16 bits of 1024 + zp
+        wd[j & 1][f] = __builtin_bit_cast(h8_t, dequant8(wq[f][j], hz | (hz << 16)));
+      }
+    };
+    auto scale = [&](int j, const f4_t (&s)[WF]) {
+#pragma unroll
+      for (int f = 0; f < WF; ++f)
+#pragma unroll
+        for (int t = 0; t < TJ; ++t) {
+#pragma unroll
+          for (int r = 0; r < 4; ++r) acc[f][t][r] = fmaf(d[j & 1][f][t][r], s[f][r], acc[f][t][r]);
+          // final here: the compiler otherwise moves every block's scaling to the chunk's end (spills)
+          asm volatile("" : "+v"(acc[f][t]));
+        }
+    };
+    read(0);
+    dequant(0);
+    f4_t sp[WF];
+#pragma unroll
+    for (int j = 0; j < 4; ++j) {
+      if (j > 0) {
+#pragma unroll
+        for (int f = 0; f < WF; ++f) sp[f] = sc[(j - 1) & 1][f];
+      }
+      if (j < 3) read(j + 1);
+      __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+      for (int t = 0; t < TJ; ++t)
+#pragma unroll
+        for (int f = 0; f < WF; ++f) d[j & 1][f][t] = mfma16x16x32(wd[j & 1][f], xf[j & 1][0][t], f4_t{0.f, 0.f, 0.f, 0.f});
+      if constexpr (SPLIT) {
+#pragma unroll
+        for (int t = 0; t < TJ; ++t)
+#pragma unroll
+          for (int f = 0; f < WF; ++f) d[j & 1][f][t] = mfma16x16x32(wd[j & 1][f], xf[j & 1][NPL - 1][t], d[j & 1][f][t]);
+      }
+      if (j < 3) dequant(j + 1);
+      if (j > 0) scale(j - 1, sp);
+      __builtin_amdgcn_sched_barrier(0);
+    }
+#pragma unroll
+    for (int f = 0; f < WF; ++f) sp[f] = sc[1][f];
+    scale(3, sp);
+  };
+  using I0 = std::integral_constant<int, 0>;
+  if constexpr (CT > 0) {
+    Wts w[CT];  // three sets live at a time
+    load_w(0, w[0]);
+    load_x(0, 0);
+    if constexpr (CT > 1) load_w(1, w[1]);
+    auto chunks = [&](auto self, auto ci) {
+      constexpr int c = decltype(ci)::value;
+      step(c, c & 1, w[c], std::integral_constant<int, c + 1 < CT ? VM_W : 0>{}, [&]() {
+        if constexpr (c + 1 < CT) load_x(c + 1, (c + 1) & 1);
+        if constexpr (c + 2 < CT) load_w(c + 2, w[c + 2]);
+      });
+      if constexpr (c + 1 < CT) self(self, std::integral_constant<int, c + 1>{});
+    };
+    chunks(chunks, I0{});
+  } else {
+    Wts wa, wb;
+    load_x(0, 0);
+    load_w(0, wa);
+    for (int c = 0; c < C; c += 2) {
+      step(c, 0, wa, I0{}, [&]() {
+        if (c + 1 < C) {
+          load_x(c + 1, 1);
+          load_w(c + 1, wb);
+        }
+      });
+      if (c + 1 < C)
+        step(c + 1, 1, wb, I0{}, [&]() {
+          if (c + 2 < C) {
+            load_x(c + 2, 0);
+            load_w(c + 2, wa);
+          }
+        });
+    }
+  }
+
+  // ---- epilogue: lane holds out[token 16 t + l16][n = n0 + (wave WF + f) 16 + 4 lg + r]
+  // RoPE: the lane's (cos, sin) entries, every load issued before the first use
+  [[maybe_unused]] f2_t cs[WF][TJ], sn[WF][TJ];
+  if constexpr (EPI == Epi::ROPE_F16) {
+#pragma unroll
+    for (int t = 0; t < TJ; ++t) {
+      const uint32_t pos = (uint32_t)(row0 + min(16 * t + l16, rows - 1)) % (uint32_t)p.seq_len;  // rows < 2^31
+#pragma unroll
+      for (int f = 0; f < WF; ++f) {
+        const uint32_t at = pos * 32 + ((ncol[f] & 63) >> 1);
+        cs[f][t] = *reinterpret_cast<const f2_t*>(p.rope_cos + at);
+        sn[f][t] = *reinterpret_cast<const f2_t*>(p.rope_sin + at);
+      }
+    }
+  }
+#pragma unroll
+  for (int f = 0; f < WF; ++f) {
+    const int n = ncol[f];
+    if (n >= p.N) continue;
+    float bv[4];
+#pragma unroll
+    for (int r = 0; r < 4; ++r) bv[r] = n + r < p.N ? wasm_h2f(braw[f][r]) : 0.0f;
+#pragma unroll
+    for (int t = 0; t < TJ; ++t) {
+      const int lt = 16 * t + l16;
+      if (lt >= rows) continue;
+      const size_t orow = (size_t)(row0 + lt);
+      float v[4];
+#pragma unroll
+      for (int r = 0; r < 4; ++r) v[r] = acc[f][t][r] + bv[r];
+      if constexpr (EPI == Epi::ROPE_F16) {
+        store_f16x4(p, orow, n, n < p.rope_cols ? rope_f16x4(v, cs[f][t], sn[f][t]) : to_f16x4(v));
+      } else {
+        store_out<EPI>(p, orow, n, v);
+      }
+    }
+  }
+}
+
+template <int WF, int BT, bool SPLIT, Epi EPI, bool GROUPED, int CT>
+void launch_k128_ct(pfhip_backend* b, const GemmArgs& a, const char* name) {
+  constexpr int BNW = 64 * WF;
+  const int t_tiles = GROUPED ? a.max_tiles : (a.M + BT - 1) / BT;
+  const long grid = (long)((a.N + BNW - 1) / BNW) * t_tiles;
+  if (grid == 0) return;
+  PF_CHECK(grid < (1L << 31), "gemm_int4: grid too large");
+  const size_t lds = (size_t)2 * (SPLIT ? 2 : 1) * BT * KC * 2 + (size_t)2 * 4 * BNW * 4;
+  const auto kern = &k_gemm_int4_k128<WF, BT, SPLIT, EPI, GROUPED, CT>;
+  allow_lds(reinterpret_cast<const void*>(kern), lds);
+  ProfScope ps(b, name);
+  hipLaunchKernelGGL(kern, dim3((unsigned)grid), dim3(256), lds, b->stream, a);
+  PF_HIP(hipGetLastError());
+}
+
+// K = 640 (the model's width) is built with its chunk count, others loop.
+template <int WF, int BT, bool SPLIT, Epi EPI, bool GROUPED>
+void launch_k128(pfhip_backend* b, const GemmArgs& a, const char* name) {
+  if (a.K == 5 * KC) return launch_k128_ct<WF, BT, SPLIT, EPI, GROUPED, 5>(b, a, name);
+  if constexpr (!GROUPED && !SPLIT && EPI == Epi::F16)
+    if (a.K == 7 * KC) return launch_k128_ct<WF, BT, SPLIT, EPI, GROUPED, 7>(b, a, name);
+  launch_k128_ct<WF, BT, SPLIT, EPI, GROUPED, 0>(b, a, name);
+}
+
+// The tiles below, for the forms that the split forward and the named
+// products use; false: not built (the kernel above takes them).
+// Dense: 32 tokens x 64 columns at every size (2048 x 1152 x 640, RoPE
+// epilogue: 21.7 us, against 24.4 with 64 x 64 and 34.7 with 64 x 128), but 64
+// tokens from 4096 rows for one fp16 plane (O projection of 8192 rows: 24.3
+// against 28.9 us).
+// Grouped: the expert plan's tile. 16 and 32 rows take 64 columns, 64 rows 128 (gate_up
+// over 13.6 rows per expert: 26.6 / 30.0 / 41.0 us on tiles of 16 / 32 / 64
+// rows; over 64: 75.7 / 66.3 / 66.3; over 256: 281 / 227 / 197).
+bool dispatch_k128(pfhip_backend* b, const GemmArgs& a, bool split, Epi epi, bool grouped, int tile_t,
+                   const char* name) {
+  if (grouped) {
+    auto tile = [&](auto wf, auto bt) {
+      constexpr int WF = decltype(wf)::value, BT = decltype(bt)::value;
+      if (epi == Epi::SWIGLU_SPLIT) {
+        if (split) launch_k128<WF, BT, true, Epi::SWIGLU_SPLIT, true>(b, a, name);
+        else launch_k128<WF, BT, false, Epi::SWIGLU_SPLIT, true>(b, a, name);
+        return true;
+      }
+      if (epi == Epi::F32 && split) {
+        launch_k128<WF, BT, true, Epi::F32, true>(b, a, name);
+        return true;
+      }
+      return false;
+    };
+    using I1 = std::integral_constant<int, 1>;
+    using I2 = std::integral_constant<int, 2>;
+    if (tile_t == 16) return tile(I1{}, std::integral_constant<int, 16>{});
+    if (tile_t == 32) return tile(I1{}, std::integral_constant<int, 32>{});
+    if (tile_t == 64) return tile(I2{}, std::integral_constant<int, 64>{});
+    return false;
+  }
+  switch (epi) {
+    case Epi::F16:
+      if (split) launch_k128<1, 32, true, Epi::F16, false>(b, a, name);
+      else if (a.M >= 4096) launch_k128<1, 64, false, Epi::F16, false>(b, a, name);
+      else launch_k128<1, 32, false, Epi::F16, false>(b, a, name);
+      return true;
+    case Epi::F32:
+      if (split) launch_k128<1, 32, true, Epi::F32, false>(b, a, name);
+      else if (a.M >= 4096) launch_k128<1, 64, false, Epi::F32, false>(b, a, name);
+      else launch_k128<1, 32, false, Epi::F32, false>(b, a, name);
+      return true;
+    case Epi::ROPE_F16:
+      if (!split) return false;
+      launch_k128<1, 32, true, Epi::ROPE_F16, false>(b, a, name);
+      return true;
+    default: return false;
+  }
+}
+
 template <int BT, bool SPLIT, bool GROUPED>
 void dispatch_epi(pfhip_backend* b, const GemmArgs& a, Epi epi, const char* name) {
   switch (epi) {
@@ -315,6 +700,11 @@ void gemm_int4(pfhip_backend* b, const GemmArgs& a, XKind xk, Epi epi, bool grou
   // slots bound every row the tile list or the row map can name)
   PF_CHECK((long)a.M * a.ldx < (1L << 31), "gemm_int4: activation offsets exceed 32 bits");
   const bool split = xk == XKind::SPLIT;
+  if (a.K % KC == 0) {
+    const bool k128 = ((reinterpret_cast<uintptr_t>(a.wz) & 1) | (reinterpret_cast<uintptr_t>(a.ws) & 3)) == 0 &&
+                      ((a.wz_gs & 1) | (a.ws_gs & 1)) == 0 && (long)a.N * a.K / 2 < (1L << 31);
+    if (k128 && dispatch_k128(b, a, split, epi, grouped, tile_t, prof_name)) return;
+  }
   if (tile_t == 64) {
     if (split) {
       if (grouped) dispatch_epi<64, true, true>(b, a, epi, prof_name);

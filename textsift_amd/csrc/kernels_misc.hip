@@ -310,9 +310,24 @@ __global__ __launch_bounds__(256) void k_add_rms_norm(const uint16_t* __restrict
 
 // ----------------------------------------------------------------------------
 // Element-wise (:969-1164).
-__global__ void k_split_f32(const float* x, uint16_t* hi, uint16_t* lo, size_t n) {
-  for (size_t i = blockIdx.x * (size_t)blockDim.x + threadIdx.x; i < n; i += (size_t)gridDim.x * blockDim.x)
-    split_hilo(x[i], hi[i], lo[i]);
+// 8 values per thread (32 bytes in, 16 + 16 out); the last n % 8 one each.
+// The planes are 16-byte aligned (scratch); x is too when vec is set.
+__global__ __launch_bounds__(256) void k_split_f32(const float* __restrict__ x, uint16_t* __restrict__ hi,
+                                                   uint16_t* __restrict__ lo, size_t n, bool vec) {
+  const size_t i = blockIdx.x * (size_t)blockDim.x + threadIdx.x;
+  const size_t n8 = vec ? n / 8 : 0;
+  if (i < n8) {
+    const f4_t a = reinterpret_cast<const f4_t*>(x)[2 * i], b = reinterpret_cast<const f4_t*>(x)[2 * i + 1];
+    uint16_t h[8], l[8];
+#pragma unroll
+    for (int r = 0; r < 8; ++r) split_hilo(r < 4 ? a[r] : b[r - 4], h[r], l[r]);
+    const u2_t h0 = pack4(h), h1 = pack4(h + 4), l0 = pack4(l), l1 = pack4(l + 4);
+    reinterpret_cast<u4_t*>(hi)[i] = u4_t{h0.x, h0.y, h1.x, h1.y};
+    reinterpret_cast<u4_t*>(lo)[i] = u4_t{l0.x, l0.y, l1.x, l1.y};
+    return;
+  }
+  const size_t j = 8 * n8 + (i - n8);
+  if (j < n) split_hilo(x[j], hi[j], lo[j]);
 }
 __global__ void k_add_f16(const uint16_t* a, const uint16_t* b, uint16_t* o, size_t n) {
   for (size_t i = blockIdx.x * (size_t)blockDim.x + threadIdx.x; i < n; i += (size_t)gridDim.x * blockDim.x)
@@ -1333,8 +1348,11 @@ void add_rms_norm_split(pfhip_backend* b, const uint16_t* a, const uint16_t* bb,
 
 void split_f32(pfhip_backend* b, const float* x, uint16_t* hi, uint16_t* lo, size_t n) {
   if (!n) return;
+  const bool vec =
+      ((reinterpret_cast<uintptr_t>(x) | reinterpret_cast<uintptr_t>(hi) | reinterpret_cast<uintptr_t>(lo)) & 15) == 0;
+  const size_t threads = vec ? n / 8 + n % 8 : n;
   ProfScope ps(b, "split_f32");
-  hipLaunchKernelGGL(k_split_f32, dim3(grid1d(n)), dim3(256), 0, b->stream, x, hi, lo, n);
+  hipLaunchKernelGGL(k_split_f32, dim3((unsigned)((threads + 255) / 256)), dim3(256), 0, b->stream, x, hi, lo, n, vec);
   PF_HIP(hipGetLastError());
 }
 
