@@ -131,3 +131,52 @@ def test_fp16_narrowing_below_normal(be, scale):
               u32s(s.size, 0, 0, 0) + struct.pack("<f", scale) + u32s(0, 0, 0)).view(np.uint16)
     ref = oracle.f32_to_fp16(s * np.float32(scale))
     assert np.array_equal(got, np.asarray(ref, np.uint16))
+
+
+# ---------------------------------------------------------------- fp16 GEMM tiles
+
+def prepared(be, q, rows, K):
+    src = [be.buffer(q[k]) for k in ("int4", "scales", "zp")]
+    out = [be.buffer(nbytes=rows * K // 2), be.buffer(nbytes=rows * (K // 32) * 4)]
+    be.dispatch("w4_prepare", src + out, u32s(rows, K, 1, 0))
+    for b in src:
+        b.release()
+    return out + [be.buffer(q["bias"])]
+
+
+@pytest.mark.parametrize("T,N,K", [(704, 1152, 640), (705, 1152, 640), (1280, 640, 896), (1281, 640, 896),
+                                   (10240, 1152, 640), (10241, 1152, 640), (10241, 640, 896), (300, 72, 256)])
+def test_matmul_w4_tile_rule(be, T, N, K):
+    """The dense tile the library chooses on each side of every line of its
+    rule gives the bits of the 64 x 64 tile."""
+    w = prepared(be, synth.qweight(1500 + N, N, K), N, K)
+    x, out = be.buffer(synth.to_fp16_bits(synth.normal(1501, T * K))), be.buffer(nbytes=T * N * 2)
+    got = []
+    for tile, wf in ((0, 0), (64, 1)):
+        be.dispatch("matmul_w4", [x] + w + [out], u32s(T, N, K, 0, tile, wf))
+        got.append(out.read(np.uint16))
+    for b in [x, out] + w:
+        b.release()
+    assert np.array_equal(got[0], got[1])
+
+
+@pytest.mark.parametrize("T", [767, 768, 1535, 1536, 10240])
+def test_moe_expert_tile_rule(be, T):
+    """The expert tile on each side of every line of its rule (16, 32, 64 and
+    128 rows) gives the bits of the 64 x 64 tile."""
+    D, E, K, F = 640, 128, 4, 640
+    rw, rb = synth.zipf_router(6, D, E)
+    fixed = [be.buffer(np.ascontiguousarray(rw.T)), be.buffer(rb)] + \
+        prepared(be, synth.qweight(1600, 2 * F, D, lead=(E,)), E * 2 * F, D) + \
+        prepared(be, synth.qweight(1601, D, F, lead=(E,)), E * D, F)
+    x = be.buffer(synth.to_fp16_bits(synth.normal(1602, T * D)))
+    outs = [be.buffer(nbytes=n) for n in (T * D * 2, T * K * 4, T * K * 4)]
+    got = []
+    for tile, wf in ((0, 0), (64, 1)):
+        be.dispatch("moe_ffn_w4", [x] + fixed + outs, u32s(T, D, E, K, F, tile, wf, 1))
+        got.append(outs[0].read(np.uint16))
+    with pytest.raises(_native.PfhipError):  # the 32-row tile is the library's own choice only
+        be.dispatch("moe_ffn_w4", [x] + fixed + outs, u32s(T, D, E, K, F, 32, 2, 1))
+    for b in [x] + fixed + outs:
+        b.release()
+    assert np.array_equal(got[0], got[1])

@@ -33,17 +33,40 @@
 using namespace pf;
 
 namespace pf {
-// Expert tile rows for the grouped GEMMs, from the mean rows per expert:
-// 128 from 256 on, 64 below, 16 (the all-K tile, fp16 numerics, K = 640 or
-// 896) below 32; fragments per wave 4, 5 and 1 respectively.
+// Expert tile rows for the grouped GEMMs, from the mean rows per expert.
+// Measured in the fp16 numerics (gate_up + down, us, 128 experts, top-4, skewed routing):
+//   rows/expert    8      16      32      64     256     375     512
+//   16 x 64      23.5   33.7    50.0    80.9   272
+//   32 x 128     24.6   32.1    42.8    56.2   156             311
+//   64 x 128     30.0   36.8    45.7    55.2   122     176     234
+//   64 x 320            43.2    56.5    67.1   138
+//   128 x 256           66.5    63.7    71.7   128     171     215
+// (with the evenly spread routing of a trained model most experts of 13.6
+// rows on average fit one 16-row tile: 29.4 against 32.8 us on 32 rows.)
+// 64 x 320, all of K at once, was the tile from 32 to 256 rows: one and a half
+// rounds of 2 workgroups per CU, against 4 per CU of the smaller tiles.
 ExpertTile expert_tile(int M, int topk, int experts, bool fp16, int D, int F) {
   const int per_expert = (int)((long)M * topk / experts);
   // split numerics, K % 128 == 0: gemm_int4's tiles of 16, 32 and 64 rows (measured there)
   if (!fp16 && D % 128 == 0 && F % 128 == 0) return {per_expert < 32 ? 16 : per_expert < 64 ? 32 : 64, 1};
-  if (per_expert >= 256) return {128, 4};
+  if (!fp16) return {per_expert >= 256 ? 128 : 64, 5};
+  if (per_expert >= 320) return {128, 4};
   const auto small_k = [](int k) { return k == 640 || k == 896; };
-  if (fp16 && small_k(D) && small_k(F) && per_expert < 32) return {16, 1};
-  return {64, 5};
+  if (small_k(D) && small_k(F) && per_expert < 24) return {16, 1};
+  return {per_expert < 48 ? 32 : 64, 2};
+}
+
+// Tile of a dense fp16-numerics GEMM without a top-k epilogue. 16 x 64 (all
+// of K at once, K = 640 or 896) while 64 x 128 tiles are fewer than 100:
+// 437 x 1152 x 640 5.9 against 7.3 us, 1024 x 1152 x 640 9.2 against 7.2. Then 64 x
+// 128, up to 10240 rows against 128 x 256 (8192 x 1152 x 640 20.9 / 24.2 us, 12000: 27.5 /
+// 25.7), and at any size where 256 columns would be padded by over an eighth (12000 x 640 x 896
+// 22.7 / 30.2 us).
+ExpertTile dense_tile(int M, int N, int K) {
+  const long tiles = (long)((M + 63) / 64) * ((N + 127) / 128);
+  if ((K == 640 || K == 896) && tiles < 100) return {16, 1};
+  const long padded = (long)((N + 255) / 256) * 256;
+  return M > 10240 && 8 * padded <= 9 * (long)N ? ExpertTile{128, 4} : ExpertTile{64, 2};
 }
 }  // namespace pf
 
@@ -268,7 +291,7 @@ struct Scr {
 // The 16-token GEMM tile loads all of K (640 or 896) at once: a workgroup
 // waits on memory once instead of once per 128-wide K chunk, which is what
 // a GEMM of a few workgroups costs. fp16 numerics only.
-constexpr int SMALL_M = 2048;           // dense GEMMs: rows up to this
+constexpr int SMALL_M = 2048;
 bool small_k(size_t K) { return K == 640 || K == 896; }
 
 int tile_for(const pfhip_model_config& c, int M) {
@@ -413,9 +436,9 @@ static void run_forward(pfhip_model* m, const int32_t* ids, const uint8_t* mask,
   const bool f16 = c.precision == PFHIP_PRECISION_FP16;
   // GEMM tiles of the fp16 path: (tokens, 16-row fragments per wave)
   const int gw_t = tt, gw_f = expert_tile(M, K, E, f16, D, F).wf;
-  // dense GEMMs of at most SMALL_M rows (O and the classifier 2x, the
-  // router 8x: measured crossovers) take the all-K 16-token tile
-  auto small_dense = [&](int k, int limit = SMALL_M) { return M <= limit && small_k((size_t)k); };
+  // the classifier up to 2 x SMALL_M rows and the router up to 8 x (measured
+  // crossovers) take the all-K 16-token tile
+  auto small_dense = [&](int k, int limit) { return M <= limit && small_k((size_t)k); };
   // O projection: one kernel with the add + norm from 16384 rows; below, the
   // O GEMM, and the add + norm either in the router GEMM (its 16-token tile
   // holds whole 640-wide rows) or as its own kernel
@@ -456,8 +479,8 @@ static void run_forward(pfhip_model* m, const int32_t* ids, const uint8_t* mask,
       a.seq_len = T; a.rope_cols = (Hq + Hkv) * hd;
       if (f16) {
         a.w = reinterpret_cast<const uint8_t*>(L.qkv4.w); a.wsz = L.qkv4.sz;
-        const bool sm = small_dense(D);
-        gemm_w4(b, a, XKind::F16, Epi::ROPE_F16, false, sm ? 16 : 128, sm ? 1 : 4, "gemm_qkv_rope");
+        const ExpertTile t = dense_tile(M, NQKV, D);
+        gemm_w4(b, a, XKind::F16, Epi::ROPE_F16, false, t.t, t.wf, "gemm_qkv_rope");
       } else {
         gemm_int4(b, a, XKind::SPLIT, Epi::ROPE_F16, false, 128, "gemm_qkv_rope");
       }
@@ -489,8 +512,8 @@ static void run_forward(pfhip_model* m, const int32_t* ids, const uint8_t* mask,
         if (fused_o) {
           gemm_w4_add_rmsnorm(b, a, h, L.ln_post, s.h2, s.xn_hi, c.eps);
         } else {
-          const bool sm = small_dense(Hq * hd, 2 * SMALL_M);
-          gemm_w4(b, a, XKind::F16, Epi::F16, false, sm ? 16 : 128, sm ? 1 : 4, "gemm_o");
+          const ExpertTile t = dense_tile(M, D, Hq * hd);
+          gemm_w4(b, a, XKind::F16, Epi::F16, false, t.t, t.wf, "gemm_o");
           if (!norm_in_router) add_rms_norm_f16(b, h, s.o, L.ln_post, s.h2, s.xn_hi, M, D, c.eps);
         }
       } else {

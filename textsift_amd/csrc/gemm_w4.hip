@@ -1037,7 +1037,7 @@ void gemm_w4(pfhip_backend* b, const GemmArgs& a, XKind xk, Epi epi, bool groupe
                  a.plan_tiles && a.plan_num_tiles && a.plan_tile_t >= 1,
              "gemm_w4: the routing plan is built by the single 16-row router tile (M <= 16), with every plan output");
   if (tile_t == 128 && wf == 4) return dispatch_grouped<4, 128>(b, g, epi, grouped, prof_name);
-  // 64-row expert tiles with K = 640 load all five chunks at once (80 KB of
+  // (64, 5) expert tiles with K = 640 load all five chunks at once (80 KB of
   // LDS, two workgroups per CU): a tile waits for memory once instead of
   // once per chunk, which is what bounds these GEMMs at a few hundred tiles
   if (tile_t == 64 && wf == 5 && grouped && a.K == 5 * KC)
@@ -1046,6 +1046,9 @@ void gemm_w4(pfhip_backend* b, const GemmArgs& a, XKind xk, Epi epi, bool groupe
   if (tile_t == 128 && wf == 2) return dispatch_grouped<2, 128>(b, g, epi, grouped, prof_name);
   if (tile_t == 64 && wf == 2) return dispatch_grouped<2, 64>(b, g, epi, grouped, prof_name);
   if (tile_t == 64 && wf == 1) return dispatch_grouped<1, 64>(b, g, epi, grouped, prof_name);
+  if (tile_t == 32 && wf == 2 && grouped && epi == Epi::SWIGLU_F16)
+    return launch<2, 32, 1, Epi::SWIGLU_F16, true, 4>(b, g, prof_name);
+  if (tile_t == 32 && wf == 2 && grouped && epi == Epi::F16) return launch<2, 32, 1, Epi::F16, true, 4>(b, g, prof_name);
   if (a.nrm_res)
     PF_CHECK(a.nrm_gamma && a.nrm_h && a.nrm_xn && a.ldx == a.K && tile_t == 16 &&
                  ((reinterpret_cast<uintptr_t>(a.nrm_res) | reinterpret_cast<uintptr_t>(a.nrm_gamma) |

@@ -162,17 +162,20 @@ void gemm_int4(pfhip_backend* b, const GemmArgs& a, XKind xk, Epi epi, bool grou
                const char* prof_name);
 
 // Tile of the grouped expert GEMMs for M tokens routed to topk of experts:
-// t tokens per tile (128, 64 or 16; also the routing plan's tile) and wf
+// t tokens per tile (128, 64, 32 or 16; also the routing plan's tile) and wf
 // 16-row weight fragments per wave (gemm_w4). The forward and the moe_ffn
 // named kernel choose it the same way.
 struct ExpertTile {
   int t, wf;
 };
 ExpertTile expert_tile(int M, int topk, int experts, bool fp16, int D, int F);
+// The same for a dense gemm_w4 product of M rows (the forward's QKV and O
+// projections and the matmul_w4 named kernel).
+ExpertTile dense_tile(int M, int N, int K);
 
 // Scale-folded int4 GEMM (gemm_w4.hip): weights prepared by w4_prepare;
 // K % 128 == 0. tile_t x wf selects the tile (BT tokens x 64*wf rows):
-// (128, 4), (128, 2), (64, 5), (64, 1), and the small-M tiles (16, 1) and
+// (128, 4), (128, 2), (64, 5), (64, 2), (64, 1), grouped (32, 2), and the small-M tiles (16, 1) and
 // (16, 2) that load all of K (640 or 896) at once.
 void gemm_w4(pfhip_backend* b, const GemmArgs& a, XKind xk, Epi epi, bool grouped, int tile_t, int wf,
              const char* prof_name);

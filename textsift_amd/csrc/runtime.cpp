@@ -241,9 +241,9 @@ static void moe_ffn_fp16(pfhip_backend* b, const uint16_t* x, const uint16_t* rw
 // chooses it for T rows when tile_t == 0.
 static void matmul_w4_auto(pfhip_backend* b, GemmArgs& a, Epi epi, int tile_t, int wf, const char* name) {
   if (tile_t == 0) {
-    const bool sm = a.M <= 2048 && (a.K == 640 || a.K == 896);
-    tile_t = sm ? 16 : 128;
-    wf = sm ? 1 : 4;
+    const ExpertTile t = dense_tile(a.M, a.N, a.K);
+    tile_t = t.t;
+    wf = t.wf;
   }
   gemm_w4(b, a, XKind::F16, epi, false, tile_t, wf, "matmul_w4");
 }
@@ -502,7 +502,7 @@ static std::vector<KernelEntry>& registry() {
                }});
   // moe_ffn_w4: moe_ffn in the fp16 numerics on prepared expert weights (BASELINE config 3 as the
   // forward runs it). push {T, D, E, K, dff, tile_t, wf, router_t} (tile_t 0: the forward's expert tile;
-  // else one of gemm_w4's grouped tiles: (128, 4), (64, 5), (64, 1), (16, 1); router_t 1: router_w is
+  // else one of gemm_w4's grouped tiles: (128, 4), (64, 5), (64, 2), (64, 1), (16, 1); router_t 1: router_w is
   // transposed, [E][D] (transpose_f16), and E == 128, K == 4: the forward's fused router chain);
   // bindings [x fp16 [T][D], router_w fp16 [D][E] (or [E][D]), router_bias fp16 [E], gu.w4, gu.sz, gu.bias,
   // dn.w4, dn.sz, dn.bias, out fp16 [T][D], routing_idx [T][K], routing_w [T][K]]
@@ -511,6 +511,7 @@ static std::vector<KernelEntry>& registry() {
                  const int F = (int)pu(p, 4);
                  PF_CHECK(T >= 1 && E >= K && K >= 1 && K <= 8, "moe_ffn_w4: bad T / E / K");
                  PF_CHECK(D % 128 == 0 && F % 128 == 0, "moe_ffn_w4: D and dff must be multiples of 128");
+                 PF_CHECK(pu(p, 5) != 32, "moe_ffn_w4: tile_t must be 0, 16, 64 or 128");
                  need(bs, 0, (size_t)T * D * 2, "moe_ffn_w4");
                  need(bs, 1, (size_t)D * E * 2, "moe_ffn_w4");
                  need(bs, 2, (size_t)E * 2, "moe_ffn_w4");
