@@ -261,6 +261,79 @@ __global__ __launch_bounds__(256) void k_embed_rms_norm4(const uint8_t* __restri
   }
 }
 
+// The same with one row per wave, for few rows: a lane holds at most two of
+// the row's 80 units instead of five of four rows', and one wave sum follows
+// instead of four, so the chain id -> table row -> sum -> store is shorter
+// and four times as many waves run it: 25 rows 10.2 -> 6.6 us, 437 rows 9.8 ->
+// 5.5, 2048 rows 10.7 -> 6.9; 8192 rows and more take the same time (bound
+// by the stores) in either form. Bit-identical: row t's units sit in the lanes
+// where k_embed_rms_norm4 has them (unit j of row t in lane (80 (t & 3) + j)
+// mod 64, lower units first), so the lanes' partial sums and their reduction
+// are the same.
+__global__ __launch_bounds__(256) void k_embed_rms_norm1(const uint8_t* __restrict__ q, const uint16_t* __restrict__ s,
+                                                         const uint8_t* __restrict__ zp,
+                                                         const int32_t* __restrict__ ids,
+                                                         const uint16_t* __restrict__ g, uint16_t* __restrict__ h,
+                                                         uint16_t* __restrict__ out, int T, int V, float eps) {
+  constexpr int D = 640, NB = D / 32, NZ = (NB + 1) / 2, UPR = D / 8;
+  const int lane = threadIdx.x & 63;
+  const int t = blockIdx.x * 4 + __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  if (t >= T) return;
+  const int id = ids[t];
+  const bool ok = id >= 0 && id < V;
+  const size_t rr = ok ? (size_t)id : 0;  // out-of-range ids read row 0, stored as 0
+  const int j0 = (lane - 16 * (t & 3)) & 63;
+  const bool two = j0 < UPR - 64;
+  const int dw[2] = {j0, two ? j0 + 64 : j0};
+  uint32_t w[2];
+  uint16_t sb[2];
+  uint8_t zb[2];
+  u4_t gw[2];
+#pragma unroll
+  for (int i = 0; i < 2; ++i) {
+    w[i] = reinterpret_cast<const uint32_t*>(q + rr * (D / 2))[dw[i]];
+    sb[i] = s[rr * NB + (dw[i] >> 2)];
+    zb[i] = zp[rr * NZ + (dw[i] >> 3)];
+    gw[i] = *reinterpret_cast<const u4_t*>(g + dw[i] * 8);
+  }
+  float v[2][8];
+  u4_t res[2];
+  float ss = 0.0f;
+#pragma unroll
+  for (int i = 0; i < 2; ++i) {
+    res[i] = u4_t{0u, 0u, 0u, 0u};
+    if (ok) {
+      const float sc = wasm_h2f(sb[i]);
+      const int z = ((dw[i] >> 2) & 1) ? (zb[i] >> 4) : (zb[i] & 0xF);
+      float e[8];
+#pragma unroll
+      for (int j = 0; j < 8; ++j) e[j] = (float)((int)((w[i] >> (4 * j)) & 0xFu) - z) * sc;
+      const u2_t a = to_f16x4_z(e), c = to_f16x4_z(e + 4);
+      res[i] = u4_t{a.x, a.y, c.x, c.y};
+    }
+    h4_to_f(u2_t{res[i].x, res[i].y}, v[i]);
+    h4_to_f(u2_t{res[i].z, res[i].w}, v[i] + 4);
+    float sq = 0.0f;
+#pragma unroll
+    for (int r = 0; r < 8; ++r) sq += v[i][r] * v[i][r];
+    ss += i == 0 || two ? sq : 0.0f;
+  }
+  const float inv = 1.0f / sqrtf(wave_sum(ss) * (1.0f / (float)D) + eps);
+#pragma unroll
+  for (int i = 0; i < 2; ++i) {
+    float gm[8], y[8];
+    h4_to_f(u2_t{gw[i].x, gw[i].y}, gm);
+    h4_to_f(u2_t{gw[i].z, gw[i].w}, gm + 4);
+#pragma unroll
+    for (int r = 0; r < 8; ++r) y[r] = v[i][r] * inv * gm[r];
+    const u2_t lo = to_f16x4_z(y), hi = to_f16x4_z(y + 4);
+    if (i == 0 || two) {
+      *reinterpret_cast<u4_t*>(h + (size_t)t * D + dw[i] * 8) = res[i];
+      *reinterpret_cast<u4_t*>(out + (size_t)t * D + dw[i] * 8) = u4_t{lo.x, lo.y, hi.x, hi.y};
+    }
+  }
+}
+
 // add_rmsnorm_fp16_to_f32 (:288-350): sum = a + b (fp16 store), sumsq of the
 // unrounded f32 sum, normalise the rounded sum.
 template <int MODE>
@@ -1280,8 +1353,12 @@ void embed_rms_norm_f16(pfhip_backend* b, const uint8_t* q, const uint16_t* s, c
   }
   if (T <= 0) return;
   ProfScope ps(b, "embed_rms_norm");
-  hipLaunchKernelGGL(k_embed_rms_norm4<5>, dim3((unsigned)((T + 15) / 16)), dim3(256), 0, b->stream, q, s, zp, ids, g,
-                     h, out, T, V, eps);
+  if (T < 8192)
+    hipLaunchKernelGGL(k_embed_rms_norm1, dim3((unsigned)((T + 3) / 4)), dim3(256), 0, b->stream, q, s, zp, ids, g, h,
+                       out, T, V, eps);
+  else
+    hipLaunchKernelGGL(k_embed_rms_norm4<5>, dim3((unsigned)((T + 15) / 16)), dim3(256), 0, b->stream, q, s, zp, ids,
+                       g, h, out, T, V, eps);
   PF_HIP(hipGetLastError());
 }
 
