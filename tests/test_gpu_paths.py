@@ -180,3 +180,39 @@ def test_moe_expert_tile_rule(be, T):
     for b in [x] + fixed + outs:
         b.release()
     assert np.array_equal(got[0], got[1])
+
+
+# ---------------------------------------------------------------- host-in / host-out staging
+
+def test_host_forward_staging(be):
+    """pfhip_model_forward through pinned staging (logits written by the
+    classifier up to 64 KiB, by a copy kernel above) and through pageable copies
+    (above 32 MiB of logits) gives the device-resident forward's bits, call after
+    call with other ids, masks and sizes (a smaller call after a larger one
+    included, and the captured and replayed forms)."""
+    from textsift_amd.config import PF_CONFIG
+    V, C = 512, PF_CONFIG.num_classes
+    m = _native.Model(be, PF_CONFIG, num_layers=1, num_experts=8, vocab_size=V)
+    for k, v in synth.make_model_weights(PF_CONFIG, seed=5, num_layers=1, num_experts=8, vocab_size=V).items():
+        m.set_weight(k, v)
+    m.finalize()
+    edge = (64 << 10) // (4 * C)  # the largest direct call: 496 rows
+    try:
+        for i, (B, T, masked) in enumerate([(1, 5, True), (1, edge, False), (1, edge + 1, True), (3, 701, True),
+                                            (1, 5, False), (1, 5, False), (1, 5, False), (125, 2048, True),
+                                            (3, 701, True), (3, 701, True), (1, edge, False)]):
+            n = B * T
+            ids = synth.token_ids(1700 + i, n, V)
+            mask = (synth.uniform(1800 + i, n) > 0.3).astype(np.uint8) if masked else np.ones(n, np.uint8)
+            got = m.forward(ids, mask, B, T)
+            ib, mb, lb = be.buffer(ids), be.buffer(mask), be.buffer(nbytes=n * C * 4)
+            m.forward_device(ib, mb if masked else None, B, T, lb)
+            ref = lb.read(np.float32)
+            for b in (ib, mb, lb):
+                b.release()
+            assert np.array_equal(got.view(np.uint32), ref.view(np.uint32)), (B, T, masked)
+        for B, T in ((0, 5), (1, 0), (2049, 2048)):  # refused before any copy
+            with pytest.raises(_native.PfhipError):
+                m.forward(np.zeros(B * T, np.int32), None, B, T)
+    finally:
+        m.close()

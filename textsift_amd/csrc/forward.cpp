@@ -127,6 +127,13 @@ struct FwdGraph {
   hipGraphExec_t exec = nullptr;
 };
 
+// Pinned host memory and its device address.
+struct HostStage {
+  void* host = nullptr;
+  void* dev = nullptr;
+  size_t size = 0;
+};
+
 struct pfhip_model {
   pfhip_backend* b = nullptr;
   pfhip_model_config cfg{};
@@ -144,10 +151,11 @@ struct pfhip_model {
   float* rope_cos = nullptr;  // fp16 table entries, widened as the reference widens them
   float* rope_sin = nullptr;
   uint16_t* rope_pairs = nullptr;  // [T][hd/2][cos, sin] fp16 bits (fp16 numerics)
-  // host-API staging
+  // host-API staging: device buffers, and pinned host memory that the GPU reads and writes directly
   pfhip_buffer* ids_buf = nullptr;
   pfhip_buffer* mask_buf = nullptr;
   pfhip_buffer* logits_buf = nullptr;
+  HostStage ids_st, mask_st, logits_st;
   // debug taps (not recorded by the allocation-free entry)
   bool taps = false;
   bool in_noalloc = false;
@@ -621,6 +629,83 @@ static void run_forward(pfhip_model* m, const int32_t* ids, const uint8_t* mask,
   if (!f16) cast_f16_f32_ieee(b, s.logits16, logits_out ? logits_out : s.logits, (size_t)M * C);
 }
 
+// The checks of a forward of batch x seq_len tokens that need no buffers; returns the rows.
+static size_t check_forward(const pfhip_model* m, uint32_t batch, uint32_t seq_len) {
+  PF_CHECK(batch >= 1 && seq_len >= 1, "batch and seq_len must be positive");
+  const size_t M = (size_t)batch * seq_len;
+  PF_CHECK(M <= (1u << 22), "batch * seq_len too large");
+  check_row_limits(m->cfg, M);
+  PF_CHECK(m->finalized, "call pfhip_model_finalize() first");
+  return M;
+}
+
+// Enqueues a forward on the backend's stream: eagerly the first time for a
+// combination of shape and buffers, captured into a graph the second time, replayed after.
+static void enqueue_forward(pfhip_model* m, const int32_t* idp, const uint8_t* mkp, int batch, int seq_len,
+                            float* lgp) {
+  if (!m->graphs || m->taps || m->b->profiling) {
+    // taps copy to the host mid-forward and profiling brackets launches
+    // with events: both run eagerly
+    run_forward(m, idp, mkp, batch, seq_len, lgp);
+    return;
+  }
+  FwdGraph* g = nullptr;
+  for (auto& e : m->graph_cache)
+    if (e.B == batch && e.T == seq_len && e.ids == idp && e.mask == mkp && e.logits == lgp) g = &e;
+  if (!g) {  // first call of this shape: eagerly (it may grow the scratch and tables, which clears the cache)
+    run_forward(m, idp, mkp, batch, seq_len, lgp);
+    if (m->graph_cache.size() >= 16) {
+      if (m->graph_cache.front().exec) hipGraphExecDestroy(m->graph_cache.front().exec);
+      m->graph_cache.erase(m->graph_cache.begin());
+    }
+    FwdGraph e;
+    e.B = batch; e.T = seq_len; e.ids = idp; e.mask = mkp; e.logits = lgp;
+    m->graph_cache.push_back(e);
+    return;
+  }
+  if (!g->exec) {  // second call: capture the launches once, then replay them
+    hipGraph_t graph = nullptr;
+    PF_HIP(hipStreamBeginCapture(m->b->stream, hipStreamCaptureModeRelaxed));
+    try {
+      run_forward(m, idp, mkp, batch, seq_len, lgp);
+    } catch (...) {
+      if (hipStreamEndCapture(m->b->stream, &graph) == hipSuccess && graph) hipGraphDestroy(graph);
+      throw;
+    }
+    PF_HIP(hipStreamEndCapture(m->b->stream, &graph));
+    const hipError_t ie = hipGraphInstantiate(&g->exec, graph, nullptr, nullptr, 0);
+    hipGraphDestroy(graph);
+    PF_HIP(ie);
+  }
+  PF_HIP(hipGraphLaunch(g->exec, m->b->stream));
+}
+
+// Grows st to at least n bytes (powers of two from 64 KiB: pinning is slow).
+// Captured forwards may name the old memory: they go with it.
+static void stage_need(pfhip_model* m, HostStage& st, size_t n) {
+  if (st.size >= n) return;
+  size_t want = 64 << 10;
+  while (want < n) want <<= 1;
+  clear_graphs(m);
+  if (st.host) {
+    PF_HIP(hipStreamSynchronize(m->b->stream));
+    hipHostFree(st.host);
+    st = HostStage{};
+  }
+  PF_HIP(hipHostMalloc(&st.host, want, hipHostMallocDefault));
+  st.size = want;
+  PF_HIP(hipHostGetDevicePointer(&st.dev, st.host, 0));
+}
+
+// pfhip_model_forward's staging. Up to STAGE_MAX bytes of logits go through
+// pinned memory kept with the model: the embedding kernel reads the ids there, the
+// logits are written there (by the classifier itself up to STAGE_DIRECT bytes,
+// whose scattered stores a copy kernel's whole lines beat above), and the
+// host waits once. Larger batches copy pageable memory, with a wait per copy.
+// 8 layers of 1 x 25 tokens: 501 -> 463 us; one layer of 12 x 1000 masked tokens: 473 -> 432.
+constexpr size_t STAGE_MAX = (size_t)32 << 20;
+constexpr size_t STAGE_DIRECT = (size_t)64 << 10;
+
 extern "C" {
 
 pfhip_model* pfhip_model_create(pfhip_backend* b, const pfhip_model_config* cfg, char* err, size_t cap) {
@@ -679,6 +764,8 @@ void pfhip_model_destroy(pfhip_model* m) {
   pfhip_release_buffer(m->b, m->ids_buf);
   pfhip_release_buffer(m->b, m->mask_buf);
   pfhip_release_buffer(m->b, m->logits_buf);
+  for (auto* st : {&m->ids_st, &m->mask_st, &m->logits_st})
+    if (st->host) hipHostFree(st->host);
   delete m;
 }
 
@@ -797,53 +884,13 @@ int pfhip_model_forward_device(pfhip_model* m, pfhip_buffer* ids, pfhip_buffer* 
                                uint32_t seq_len, pfhip_buffer* logits, char* err, size_t cap) {
   try {
     PF_CHECK(m && ids && logits, "null argument");
-    PF_CHECK(batch >= 1 && seq_len >= 1, "batch and seq_len must be positive");
-    const size_t M = (size_t)batch * seq_len;
-    PF_CHECK(M <= (1u << 22), "batch * seq_len too large");
-    check_row_limits(m->cfg, M);
-    PF_CHECK(m->finalized, "call pfhip_model_finalize() first");
+    const size_t M = check_forward(m, batch, seq_len);
     PF_CHECK(ids->size >= M * 4, "ids buffer too small");
     PF_CHECK(!mask || mask->size >= M, "mask buffer too small");
     PF_CHECK(logits->size >= M * m->cfg.classes * 4, "logits buffer too small");
     PF_HIP(hipSetDevice(m->b->device));
-    const int32_t* idp = static_cast<const int32_t*>(ids->ptr);
-    const uint8_t* mkp = mask ? static_cast<const uint8_t*>(mask->ptr) : nullptr;
-    float* lgp = static_cast<float*>(logits->ptr);
-    if (!m->graphs || m->taps || m->b->profiling) {
-      // taps copy to the host mid-forward and profiling brackets launches
-      // with events: both run eagerly
-      run_forward(m, idp, mkp, (int)batch, (int)seq_len, lgp);
-    } else {
-      FwdGraph* g = nullptr;
-      for (auto& e : m->graph_cache)
-        if (e.B == (int)batch && e.T == (int)seq_len && e.ids == idp && e.mask == mkp && e.logits == lgp) g = &e;
-      if (!g) {  // first call of this shape: eagerly (it may grow the scratch and tables, which clears the cache)
-        run_forward(m, idp, mkp, (int)batch, (int)seq_len, lgp);
-        if (m->graph_cache.size() >= 16) {
-          if (m->graph_cache.front().exec) hipGraphExecDestroy(m->graph_cache.front().exec);
-          m->graph_cache.erase(m->graph_cache.begin());
-        }
-        FwdGraph e;
-        e.B = (int)batch; e.T = (int)seq_len; e.ids = idp; e.mask = mkp; e.logits = lgp;
-        m->graph_cache.push_back(e);
-      } else {
-        if (!g->exec) {  // second call: capture the launches once, then replay them
-          hipGraph_t graph = nullptr;
-          PF_HIP(hipStreamBeginCapture(m->b->stream, hipStreamCaptureModeRelaxed));
-          try {
-            run_forward(m, idp, mkp, (int)batch, (int)seq_len, lgp);
-          } catch (...) {
-            if (hipStreamEndCapture(m->b->stream, &graph) == hipSuccess && graph) hipGraphDestroy(graph);
-            throw;
-          }
-          PF_HIP(hipStreamEndCapture(m->b->stream, &graph));
-          const hipError_t ie = hipGraphInstantiate(&g->exec, graph, nullptr, nullptr, 0);
-          hipGraphDestroy(graph);
-          PF_HIP(ie);
-        }
-        PF_HIP(hipGraphLaunch(g->exec, m->b->stream));
-      }
-    }
+    enqueue_forward(m, static_cast<const int32_t*>(ids->ptr), mask ? static_cast<const uint8_t*>(mask->ptr) : nullptr,
+                    (int)batch, (int)seq_len, static_cast<float*>(logits->ptr));
     PF_HIP(hipStreamSynchronize(m->b->stream));
     prof_flush(m->b);
     return 0;
@@ -857,11 +904,7 @@ int pfhip_model_forward_device_noalloc(pfhip_model* m, pfhip_buffer* ids, pfhip_
                                        uint32_t seq_len, pfhip_buffer* logits, char* err, size_t cap) {
   try {
     PF_CHECK(m && ids && logits, "null argument");
-    PF_CHECK(batch >= 1 && seq_len >= 1, "batch and seq_len must be positive");
-    const size_t M = (size_t)batch * seq_len;
-    PF_CHECK(M <= (1u << 22), "batch * seq_len too large");
-    check_row_limits(m->cfg, M);
-    PF_CHECK(m->finalized, "call pfhip_model_finalize() first");
+    const size_t M = check_forward(m, batch, seq_len);
     PF_CHECK(ids->size >= M * 4, "ids buffer too small");
     PF_CHECK(!mask || mask->size >= M, "mask buffer too small");
     PF_CHECK(logits->size >= M * m->cfg.classes * 4, "logits buffer too small");
@@ -889,19 +932,17 @@ int pfhip_model_forward(pfhip_model* m, const int32_t* ids, const uint8_t* mask,
                         float* logits, char* err, size_t cap) {
   try {
     PF_CHECK(m && ids && logits, "null argument");
-    PF_CHECK(batch >= 1 && seq_len >= 1, "batch and seq_len must be positive");
-    const size_t M = (size_t)batch * seq_len;
+    const size_t M = check_forward(m, batch, seq_len);
+    PF_HIP(hipSetDevice(m->b->device));
     char e2[PFHIP_ERR_CAP];
     auto ensure = [&](pfhip_buffer*& buf, size_t bytes) {
+      bytes = al256(bytes);
       if (!buf || buf->size < bytes) {
         pfhip_release_buffer(m->b, buf);
         buf = pfhip_create_empty_buffer(m->b, bytes, e2, sizeof e2);
         PF_CHECK(buf, e2);
       }
     };
-    ensure(m->ids_buf, M * 4);
-    ensure(m->logits_buf, M * m->cfg.classes * 4);
-    PF_CHECK(pfhip_write_buffer(m->b, m->ids_buf, 0, ids, M * 4, e2, sizeof e2) == 0, e2);
     // wasm.ts:753-764: an all-ones mask is elided
     bool use_mask = false;
     if (mask)
@@ -910,14 +951,36 @@ int pfhip_model_forward(pfhip_model* m, const int32_t* ids, const uint8_t* mask,
           use_mask = true;
           break;
         }
-    if (use_mask) {
-      ensure(m->mask_buf, M);
-      PF_CHECK(pfhip_write_buffer(m->b, m->mask_buf, 0, mask, M, e2, sizeof e2) == 0, e2);
+    const size_t lbytes = M * m->cfg.classes * 4;
+    if (use_mask) ensure(m->mask_buf, M);
+    if (lbytes > STAGE_MAX) {
+      ensure(m->ids_buf, M * 4);
+      ensure(m->logits_buf, lbytes);
+      PF_CHECK(pfhip_write_buffer(m->b, m->ids_buf, 0, ids, M * 4, e2, sizeof e2) == 0, e2);
+      if (use_mask) PF_CHECK(pfhip_write_buffer(m->b, m->mask_buf, 0, mask, M, e2, sizeof e2) == 0, e2);
+      PF_CHECK(pfhip_model_forward_device(m, m->ids_buf, use_mask ? m->mask_buf : nullptr, batch, seq_len,
+                                          m->logits_buf, e2, sizeof e2) == 0,
+               e2);
+      PF_CHECK(pfhip_read_buffer(m->b, m->logits_buf, 0, logits, lbytes, e2, sizeof e2) == 0, e2);
+      return 0;
     }
-    PF_CHECK(pfhip_model_forward_device(m, m->ids_buf, use_mask ? m->mask_buf : nullptr, batch, seq_len,
-                                        m->logits_buf, e2, sizeof e2) == 0,
-             e2);
-    PF_CHECK(pfhip_read_buffer(m->b, m->logits_buf, 0, logits, M * m->cfg.classes * 4, e2, sizeof e2) == 0, e2);
+    const bool direct = lbytes <= STAGE_DIRECT;
+    if (!direct) ensure(m->logits_buf, lbytes);
+    stage_need(m, m->ids_st, M * 4);
+    stage_need(m, m->logits_st, al256(lbytes));
+    memcpy(m->ids_st.host, ids, M * 4);
+    if (use_mask) {  // read by every layer's attention: copied to the device
+      stage_need(m, m->mask_st, al256(M));
+      memcpy(m->mask_st.host, mask, M);
+      copy16(m->b, m->mask_st.dev, m->mask_buf->ptr, (M + 15) & ~(size_t)15);
+    }
+    enqueue_forward(m, static_cast<const int32_t*>(m->ids_st.dev),
+                    use_mask ? static_cast<const uint8_t*>(m->mask_buf->ptr) : nullptr, (int)batch, (int)seq_len,
+                    static_cast<float*>(direct ? m->logits_st.dev : m->logits_buf->ptr));
+    if (!direct) copy16(m->b, m->logits_buf->ptr, m->logits_st.dev, (lbytes + 15) & ~(size_t)15);
+    PF_HIP(hipStreamSynchronize(m->b->stream));
+    prof_flush(m->b);
+    memcpy(logits, m->logits_st.host, lbytes);
     return 0;
   } catch (const std::exception& ex) {
     set_err(err, cap, ex.what());

@@ -1284,7 +1284,7 @@ void copy16(pfhip_backend* b, const void* src, void* dst, size_t bytes) {
            "copy16: 16-byte aligned sizes and pointers");
   if (!bytes) return;
   ProfScope ps(b, "copy16");
-  hipLaunchKernelGGL(k_copy16, dim3(4096), dim3(256), 0, b->stream, static_cast<const u4_t*>(src),
+  hipLaunchKernelGGL(k_copy16, dim3((unsigned)std::min<size_t>(4096, (bytes / 16 + 255) / 256)), dim3(256), 0, b->stream, static_cast<const u4_t*>(src),
                      static_cast<u4_t*>(dst), bytes / 16);
   PF_HIP(hipGetLastError());
 }
