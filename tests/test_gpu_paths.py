@@ -216,3 +216,36 @@ def test_host_forward_staging(be):
                 m.forward(np.zeros(B * T, np.int32), None, B, T)
     finally:
         m.close()
+
+
+# ---------------------------------------------------------------- routing plan
+
+@pytest.mark.parametrize("T,E,tile_rows", [(255, 128, 0), (256, 200, 0), (257, 128, 0), (1025, 128, 16), (4097, 37, 64),
+                                           (16383, 128, 16), (16384, 128, 64), (1300, 128, 512)])
+def test_routing_plan_block_sizes(be, T, E, tile_rows):
+    """The plan on each side of its block-size rule (256- and 1024-token
+    blocks; tile_rows 0: the single-block plan, else from tile counts): expert offsets,
+    slots and tiles equal a stable sort by expert, bit for bit."""
+    K, tt = 4, 64
+    r = np.random.RandomState(T)
+    idx = np.argsort(r.rand(T, E) * np.linspace(1, 3, E), axis=1)[:, :K].astype(np.int32)
+    order = np.argsort(idx.ravel(), kind="stable")
+    cnt = np.bincount(idx.ravel(), minlength=E)
+    off = np.concatenate([[0], np.cumsum(cnt)]).astype(np.int32)
+    slot_of = np.empty(T * K, np.int32)
+    slot_of[order] = np.arange(T * K)
+    tiles = [(e, off[e] + i, min(tt, cnt[e] - i), 0) for e in range(E) for i in range(0, cnt[e], tt)]
+    ins = [be.buffer(idx)]
+    if tile_rows:
+        counts = np.stack([np.bincount(idx[i:i + tile_rows].ravel(), minlength=E) for i in range(0, T, tile_rows)])
+        ins.append(be.buffer(counts.astype(np.int32)))
+    outs = [be.buffer(nbytes=n) for n in ((E + 1) * 4, T * K * 4, T * K * 4, (T * K // tt + 1 + E) * 16, 4)]
+    if tile_rows:
+        be.dispatch("moe_route_counts", ins + outs, u32s(T, K, E, tt, tile_rows))
+    else:
+        be.dispatch("moe_route", ins + outs, u32s(T, K, E, tt))
+    got = [o.read(np.int32) for o in outs]
+    for b in ins + outs:
+        b.release()
+    assert np.array_equal(got[0], off) and np.array_equal(got[1], order // K) and np.array_equal(got[2], slot_of)
+    assert got[4][0] == len(tiles) and np.array_equal(got[3][:4 * len(tiles)], np.array(tiles, np.int32).ravel())

@@ -7,6 +7,7 @@
 #include "epilogue.h"
 #include "pfhip_internal.h"
 #include "topk.h"
+#include <type_traits>
 #include "combine.h"
 
 namespace pf {
@@ -534,6 +535,11 @@ __global__ __launch_bounds__(256) void k_router_topk(const float* __restrict__ l
 // pairs with expert e in ascending token order: browser/inference/
 // expert.ts:125-145). Deterministic: no atomics anywhere.
 constexpr int RBLK = 1024;          // tokens per counting block
+// The same for the single-kernel plans of few tokens: a quarter of the waves per
+// barrier and of the serial loops over bitmap words and partial sums. 25 tokens
+// 5.0 -> 4.3 us, 2048 10.2 -> 6.2, 12000 13.5 -> 11.8; 32768 11.7 -> 12.3
+// (every block sums all tile counts), so 1024-token blocks from 16384 on.
+constexpr int SMALL_RBLK = 256;
 constexpr int BWS = RBLK / 32 + 1;  // bitmap words per expert in LDS (padded: rows in distinct banks)
 
 // Per-block expert bitmaps: bit t of bits[e][t / 32] is set when token t of
@@ -548,14 +554,16 @@ __device__ __forceinline__ void moe_load_ids(const int32_t* __restrict__ idx, in
   for (int k = 0; k < MAXK; ++k) ids[k] = (k < K && tl < nt) ? idx[(size_t)(t0 + tl) * K + k] : -1;
 }
 
+template <int RB = RBLK>
 __device__ __forceinline__ void moe_block_bitmap_ids(const int (&ids)[MAXK], uint32_t* bits, int E) {
-  for (int i = threadIdx.x; i < E * BWS; i += blockDim.x) bits[i] = 0u;
+  constexpr int BW = RB / 32 + 1;
+  for (int i = threadIdx.x; i < E * BW; i += RB) bits[i] = 0u;
   __syncthreads();
   const int tl = threadIdx.x;
 #pragma unroll
   for (int k = 0; k < MAXK; ++k) {
     const int e = ids[k];
-    if ((unsigned)e < (unsigned)E) atomicOr(&bits[e * BWS + (tl >> 5)], 1u << (tl & 31));
+    if ((unsigned)e < (unsigned)E) atomicOr(&bits[e * BW + (tl >> 5)], 1u << (tl & 31));
   }
   __syncthreads();
 }
@@ -569,15 +577,17 @@ __device__ __forceinline__ void moe_block_bitmap(const int32_t* __restrict__ idx
 
 // pre[e][w] = tokens of the block routed to e among words 0 .. w-1 of the
 // bitmap (so a token's rank is pre[e][w] plus a popcount within its word)
+template <int RB = RBLK>
 __device__ __forceinline__ void moe_word_prefix(const uint32_t* bits, uint16_t* pre, int E) {
-  for (int e = threadIdx.x; e < E; e += blockDim.x) {
-    uint32_t w[RBLK / 32];
+  constexpr int BW = RB / 32 + 1;
+  for (int e = threadIdx.x; e < E; e += RB) {
+    uint32_t w[RB / 32];
 #pragma unroll
-    for (int u = 0; u < RBLK / 32; ++u) w[u] = bits[e * BWS + u];
+    for (int u = 0; u < RB / 32; ++u) w[u] = bits[e * BW + u];
     int run = 0;
 #pragma unroll
-    for (int u = 0; u < RBLK / 32; ++u) {
-      pre[e * BWS + u] = (uint16_t)run;
+    for (int u = 0; u < RB / 32; ++u) {
+      pre[e * BW + u] = (uint16_t)run;
       run += __popc(w[u]);
     }
   }
@@ -778,23 +788,25 @@ __global__ __launch_bounds__(RBLK) void k_moe_scatter(const int32_t* __restrict_
 // experts (rows and tiles) and the slot assignment. Same outputs as the
 // three kernels (expert_off, slot_token, slot_of, tiles, num_tiles; counts
 // and blk_off are not written: nothing else reads them).
-__global__ __launch_bounds__(RBLK) void k_moe_route_small(const int32_t* __restrict__ idx,
+template <int RB>
+__global__ __launch_bounds__(RB) void k_moe_route_small(const int32_t* __restrict__ idx,
                                                           int32_t* __restrict__ expert_off,
                                                           int32_t* __restrict__ slot_token,
                                                           int32_t* __restrict__ slot_of, int32_t* __restrict__ tiles,
                                                           int32_t* __restrict__ num_tiles, int T, int K, int E,
                                                           int tile_t) {
-  __shared__ uint32_t bits[256 * BWS];
-  __shared__ int32_t off[256], toff[256], wsum[2][RBLK / 64];
+  constexpr int BW = RB / 32 + 1;
+  __shared__ uint32_t bits[256 * BW];
+  __shared__ int32_t off[256], toff[256], wsum[2][RB / 64];
   int ids[MAXK];  // this thread's token's expert ids, read once
   moe_load_ids(idx, 0, T, K, ids);
-  moe_block_bitmap_ids(ids, bits, E);
+  moe_block_bitmap_ids<RB>(ids, bits, E);
   const int tid = threadIdx.x, lane = tid & 63, wv = tid >> 6;
   // rows c and tiles n of expert e = tid; inclusive scans within the wave
   int c = 0;
   if (tid < E) {
 #pragma unroll
-    for (int w = 0; w < RBLK / 32; ++w) c += __popc(bits[tid * BWS + w]);
+    for (int w = 0; w < RB / 32; ++w) c += __popc(bits[tid * BW + w]);
   }
   const int n = (c + tile_t - 1) / tile_t;
   int ci = c, ni = n;
@@ -813,7 +825,7 @@ __global__ __launch_bounds__(RBLK) void k_moe_route_small(const int32_t* __restr
   __syncthreads();
   int cb = 0, nbase = 0, ct = 0, nt = 0;
 #pragma unroll
-  for (int w = 0; w < RBLK / 64; ++w) {
+  for (int w = 0; w < RB / 64; ++w) {
     cb += w < wv ? wsum[0][w] : 0;
     nbase += w < wv ? wsum[1][w] : 0;
     ct += wsum[0][w];
@@ -831,8 +843,8 @@ __global__ __launch_bounds__(RBLK) void k_moe_route_small(const int32_t* __restr
   }
   __syncthreads();
   moe_write_tiles(toff, off, ct, E, nt, tile_t, tiles);
-  __shared__ uint16_t pre[256 * BWS];
-  moe_word_prefix(bits, pre, E);
+  __shared__ uint16_t pre[256 * BW];
+  moe_word_prefix<RB>(bits, pre, E);
   if (tid >= T) return;
   const int wl = tid >> 5;
   const uint32_t below = (1u << (tid & 31)) - 1u;
@@ -841,7 +853,7 @@ __global__ __launch_bounds__(RBLK) void k_moe_route_small(const int32_t* __restr
     const int e = ids[k];
     if ((unsigned)e >= (unsigned)E) continue;
     const size_t i = (size_t)tid * K + k;
-    const int rank = pre[e * BWS + wl] + __popc(bits[e * BWS + wl] & below);
+    const int rank = pre[e * BW + wl] + __popc(bits[e * BW + wl] & below);
     const int pos = off[e] + rank;
     slot_token[pos] = tid;
     slot_of[i] = pos;
@@ -856,18 +868,20 @@ __global__ __launch_bounds__(RBLK) void k_moe_route_small(const int32_t* __restr
 // within the expert), scans the totals over experts, and assigns its tokens'
 // slots by bitmap ranks as k_moe_scatter does. Block 0 also writes
 // expert_off, the tile list and num_tiles. Same outputs as the three kernels.
-__global__ __launch_bounds__(RBLK) void k_moe_route_counts(const int32_t* __restrict__ idx,
+template <int RB>
+__global__ __launch_bounds__(RB) void k_moe_route_counts(const int32_t* __restrict__ idx,
                                                            const int32_t* __restrict__ counts, int n_ct,
                                                            int ct_per_blk, int32_t* __restrict__ expert_off,
                                                            int32_t* __restrict__ slot_token,
                                                            int32_t* __restrict__ slot_of, int32_t* __restrict__ tiles,
                                                            int32_t* __restrict__ num_tiles, int T, int K, int E,
                                                            int tile_t) {
-  __shared__ uint32_t bits[256 * BWS];
-  __shared__ int32_t psum[2][4 * RBLK];  // per (part of the tiles, expert): all tiles, tiles before the block
-  __shared__ int32_t off[256], ebase[256], toff[256], wsum[2][RBLK / 64];
-  __shared__ uint16_t pre[256 * BWS];
-  const int blk = blockIdx.x, t0 = blk * RBLK, ntok = min(RBLK, T - t0);
+  constexpr int BW = RB / 32 + 1;
+  __shared__ uint32_t bits[256 * BW];
+  __shared__ int32_t psum[2][4 * RB];  // per (part of the tiles, expert): all tiles, tiles before the block
+  __shared__ int32_t off[256], ebase[256], toff[256], wsum[2][RB / 64];
+  __shared__ uint16_t pre[256 * BW];
+  const int blk = blockIdx.x, t0 = blk * RB, ntok = min(RB, T - t0);
   const int tid = threadIdx.x, lane = tid & 63, wv = tid >> 6;
   // this thread's token's expert ids, issued before the count loads so both
   // latencies overlap, and kept for the slot assignment
@@ -875,13 +889,13 @@ __global__ __launch_bounds__(RBLK) void k_moe_route_counts(const int32_t* __rest
   moe_load_ids(idx, t0, ntok, K, ids);
   // Per-expert sums over the tiles, in G parts of the tile range. With E a
   // multiple of 4 a thread loads 16 bytes (4 experts' counts) per tile:
-  // E2 / 4 expert groups x G = 4 RBLK / E2 parts; otherwise one expert per
-  // thread: E2 experts x G = RBLK / E2 parts (E2: E rounded up to 64, 128 or
+  // E2 / 4 expert groups x G = 4 RB / E2 parts; otherwise one expert per
+  // thread: E2 experts x G = RB / E2 parts (E2: E rounded up to 64, 128 or
   // 256). Loads are issued 16 at a time with addresses clamped into the
   // array and values past the range dropped.
   const int E2 = E <= 64 ? 64 : (E <= 128 ? 128 : 256);
   const bool vec = (E & 3) == 0;
-  const int G = vec ? 4 * RBLK / E2 : RBLK / E2;
+  const int G = vec ? 4 * RB / E2 : RB / E2;
   {
     const int tb = blk * ct_per_blk;
     const int lanes = vec ? E2 / 4 : E2;  // threads per part
@@ -928,7 +942,7 @@ __global__ __launch_bounds__(RBLK) void k_moe_route_counts(const int32_t* __rest
       psum[1][q * E2 + e0] = sb[0];
     }
   }
-  moe_block_bitmap_ids(ids, bits, E);  // (its barriers also publish psum)
+  moe_block_bitmap_ids<RB>(ids, bits, E);  // (its barriers also publish psum)
   // rows c and tiles n of expert e = tid; inclusive scans within the wave
   int c = 0, below = 0;
   if (tid < E) {
@@ -954,7 +968,7 @@ __global__ __launch_bounds__(RBLK) void k_moe_route_counts(const int32_t* __rest
   __syncthreads();
   int cb = 0, nbase = 0, ct = 0, nt = 0;
 #pragma unroll
-  for (int w = 0; w < RBLK / 64; ++w) {
+  for (int w = 0; w < RB / 64; ++w) {
     cb += w < wv ? wsum[0][w] : 0;
     nbase += w < wv ? wsum[1][w] : 0;
     ct += wsum[0][w];
@@ -973,7 +987,7 @@ __global__ __launch_bounds__(RBLK) void k_moe_route_counts(const int32_t* __rest
   }
   __syncthreads();
   if (blk == 0) moe_write_tiles(toff, ebase, ct, E, nt, tile_t, tiles);
-  moe_word_prefix(bits, pre, E);
+  moe_word_prefix<RB>(bits, pre, E);
   if (tid >= ntok) return;
   const int wl = tid >> 5;
   const uint32_t lower = (1u << (tid & 31)) - 1u;
@@ -982,7 +996,7 @@ __global__ __launch_bounds__(RBLK) void k_moe_route_counts(const int32_t* __rest
     const int e = ids[k];
     if ((unsigned)e >= (unsigned)E) continue;
     const size_t i = (size_t)(t0 + tid) * K + k;
-    const int rank = pre[e * BWS + wl] + __popc(bits[e * BWS + wl] & lower);
+    const int rank = pre[e * BW + wl] + __popc(bits[e * BW + wl] & lower);
     const int pos = off[e] + rank;
     slot_token[pos] = t0 + tid;
     slot_of[i] = pos;
@@ -1528,8 +1542,13 @@ void moe_route(pfhip_backend* b, const int32_t* idx, int T, int K, int E, const 
   const int nblk = (T + RBLK - 1) / RBLK;
   if (nblk == 1) {
     ProfScope ps(b, "moe_route");
-    hipLaunchKernelGGL(k_moe_route_small, dim3(1), dim3(RBLK), 0, b->stream, idx, m.expert_off, m.slot_token,
-                       m.slot_of, m.tiles, m.num_tiles, T, K, E, m.tile_t);
+    auto go = [&](auto rb) {
+      constexpr int RB = decltype(rb)::value;
+      hipLaunchKernelGGL(k_moe_route_small<RB>, dim3(1), dim3(RB), 0, b->stream, idx, m.expert_off, m.slot_token,
+                         m.slot_of, m.tiles, m.num_tiles, T, K, E, m.tile_t);
+    };
+    if (T <= SMALL_RBLK) go(std::integral_constant<int, SMALL_RBLK>{});
+    else go(std::integral_constant<int, RBLK>{});
     PF_HIP(hipGetLastError());
     return;
   }
@@ -1560,10 +1579,15 @@ void moe_route_counts(pfhip_backend* b, const int32_t* idx, const int32_t* count
   PF_CHECK(tile_rows >= 1 && RBLK % tile_rows == 0, "moe_route_counts: the count tiles must divide 1024 rows");
   PF_CHECK(counts, "moe_route_counts: null counts");
   if (T <= 0) return;
-  const int nblk = (T + RBLK - 1) / RBLK, n_ct = (T + tile_rows - 1) / tile_rows;
+  const int n_ct = (T + tile_rows - 1) / tile_rows;
   ProfScope ps(b, "moe_route");
-  hipLaunchKernelGGL(k_moe_route_counts, dim3(nblk), dim3(RBLK), 0, b->stream, idx, counts, n_ct, RBLK / tile_rows,
-                     m.expert_off, m.slot_token, m.slot_of, m.tiles, m.num_tiles, T, K, E, m.tile_t);
+  auto go = [&](auto rb) {
+    constexpr int RB = decltype(rb)::value;
+    hipLaunchKernelGGL(k_moe_route_counts<RB>, dim3((T + RB - 1) / RB), dim3(RB), 0, b->stream, idx, counts, n_ct,
+                       RB / tile_rows, m.expert_off, m.slot_token, m.slot_of, m.tiles, m.num_tiles, T, K, E, m.tile_t);
+  };
+  if (T < 16384 && SMALL_RBLK % tile_rows == 0) go(std::integral_constant<int, SMALL_RBLK>{});
+  else go(std::integral_constant<int, RBLK>{});
   PF_HIP(hipGetLastError());
 }
 
