@@ -221,11 +221,12 @@ def test_host_forward_staging(be):
 # ---------------------------------------------------------------- routing plan
 
 @pytest.mark.parametrize("T,E,tile_rows", [(255, 128, 0), (256, 200, 0), (257, 128, 0), (1025, 128, 16), (4097, 37, 64),
-                                           (16383, 128, 16), (16384, 128, 64), (1300, 128, 512)])
+                                           (16383, 128, 16), (16384, 128, 64), (1300, 128, 512), (1025, 256, 0),
+                                           (65535, 64, 0), (65536, 64, 0)])
 def test_routing_plan_block_sizes(be, T, E, tile_rows):
-    """The plan on each side of its block-size rule (256- and 1024-token
-    blocks; tile_rows 0: the single-block plan, else from tile counts): expert offsets,
-    slots and tiles equal a stable sort by expert, bit for bit."""
+    """The plan on each side of its rules (256- and 1024-token blocks; tile_rows
+    0: from the picks alone, in one, two or three kernels, else from tile counts):
+    expert offsets, slots and tiles equal a stable sort by expert, bit for bit."""
     K, tt = 4, 64
     r = np.random.RandomState(T)
     idx = np.argsort(r.rand(T, E) * np.linspace(1, 3, E), axis=1)[:, :K].astype(np.int32)

@@ -345,10 +345,6 @@ size_t scratch_layout(const pfhip_model_config& c, int M, Scr* s, void* base) {
 
 }  // namespace
 
-namespace pf {
-void cast_f16_f32_ieee(pfhip_backend* b, const uint16_t* s, float* d, size_t n);
-}
-
 static void record_tap(pfhip_model* m, const std::string& name, const void* dev, size_t bytes) {
   if (!m->taps || m->in_noalloc) return;
   std::vector<uint8_t>& v = m->tap[name];
@@ -613,20 +609,18 @@ static void run_forward(pfhip_model* m, const int32_t* ids, const uint8_t* mask,
     QW sc = qw(m, "score");
     a.w = sc.q; a.ws = sc.s; a.wz = sc.z; a.bias = sc.bias;
     a.out = s.logits16; a.ldo = C; a.M = M; a.N = C; a.K = D;
+    // wasm.ts:776-796 widens the fp16 logits IEEE-correctly: the epilogue
+    // stores them widened (the fp16 copy only for the taps)
+    a.out_f32w = logits_out ? logits_out : s.logits;
+    if (!m->taps) a.out = nullptr;
     if (f16) {
       a.w = reinterpret_cast<const uint8_t*>(m->score4.w); a.wsz = m->score4.sz;
-      // wasm.ts:776-796 widens the fp16 logits IEEE-correctly: the epilogue
-      // stores them widened (the fp16 copy only for the taps)
-      a.out_f32w = logits_out ? logits_out : s.logits;
-      if (!m->taps) a.out = nullptr;
       gemm_w4(b, a, XKind::F16, Epi::F16, false, small_dense(D, 2 * SMALL_M) ? 16 : 64, 1, "gemm_classifier");
     } else {
       gemm_int4(b, a, XKind::SPLIT, Epi::F16, false, 128, "gemm_classifier");
     }
   }
   record_tap(m, "logits16", s.logits16, (size_t)M * C * 2);
-  // wasm.ts:776-796 widens the fp16 logits IEEE-correctly
-  if (!f16) cast_f16_f32_ieee(b, s.logits16, logits_out ? logits_out : s.logits, (size_t)M * C);
 }
 
 // The checks of a forward of batch x seq_len tokens that need no buffers; returns the rows.

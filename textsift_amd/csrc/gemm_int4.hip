@@ -681,7 +681,8 @@ void gemm_int4(pfhip_backend* b, const GemmArgs& a, XKind xk, Epi epi, bool grou
                const char* prof_name) {
   PF_CHECK(a.K > 0 && a.K % 32 == 0, "gemm_int4: K must be a positive multiple of 32");
   PF_CHECK(a.N > 0, "gemm_int4: N must be positive");
-  PF_CHECK(a.x && a.w && a.ws && a.out, "gemm_int4: null operand");
+  PF_CHECK(a.x && a.w && a.ws && (a.out || a.out_f32w), "gemm_int4: null operand");
+  if (a.out_f32w) PF_CHECK(epi == Epi::F16 && !grouped, "gemm_int4: the widened f32 output is for the dense F16 epilogue");
   PF_CHECK(a.ldx % 8 == 0 && a.K % 8 == 0, "gemm_int4: activation row stride must allow 16-byte loads");
   PF_CHECK((reinterpret_cast<uintptr_t>(a.x) & 15) == 0 && (reinterpret_cast<uintptr_t>(a.w) & 15) == 0,
            "gemm_int4: activations and weights must be 16-byte aligned");

@@ -411,10 +411,6 @@ __global__ void k_cast_f16_f32(const uint16_t* s, float* d, size_t n) {
   for (size_t i = blockIdx.x * (size_t)blockDim.x + threadIdx.x; i < n; i += (size_t)gridDim.x * blockDim.x)
     d[i] = wasm_h2f(s[i]);
 }
-__global__ void k_cast_f16_f32_ieee(const uint16_t* s, float* d, size_t n) {
-  for (size_t i = blockIdx.x * (size_t)blockDim.x + threadIdx.x; i < n; i += (size_t)gridDim.x * blockDim.x)
-    d[i] = hw_h2f(s[i]);
-}
 __global__ void k_cast_f32_f16_scaled(const float* s, uint16_t* d, size_t n, float scale) {
   for (size_t i = blockIdx.x * (size_t)blockDim.x + threadIdx.x; i < n; i += (size_t)gridDim.x * blockDim.x)
     d[i] = wasm_f2h(s[i] * scale);
@@ -615,16 +611,20 @@ __device__ __forceinline__ void moe_write_tiles(const int32_t* tile0, const int3
 }
 
 // counts[blk][e] = tokens of block blk routed to expert e.
-__global__ __launch_bounds__(RBLK) void k_moe_count(const int32_t* __restrict__ idx, int32_t* __restrict__ counts,
+template <int RB>
+__global__ __launch_bounds__(RB) void k_moe_count(const int32_t* __restrict__ idx, int32_t* __restrict__ counts,
                                                     int T, int K, int E) {
-  __shared__ uint32_t bits[256 * BWS];
+  constexpr int BW = RB / 32 + 1;
+  __shared__ uint32_t bits[256 * BW];
   const int blk = blockIdx.x;
-  const int t0 = blk * RBLK;
-  moe_block_bitmap(idx, bits, t0, min(RBLK, T - t0), K, E);
+  const int t0 = blk * RB;
+  int ids[MAXK];
+  moe_load_ids(idx, t0, min(RB, T - t0), K, ids);
+  moe_block_bitmap_ids<RB>(ids, bits, E);
   for (int e = threadIdx.x; e < E; e += blockDim.x) {
     int c = 0;
 #pragma unroll
-    for (int w = 0; w < RBLK / 32; ++w) c += __popc(bits[e * BWS + w]);
+    for (int w = 0; w < RB / 32; ++w) c += __popc(bits[e * BW + w]);
     counts[(size_t)blk * E + e] = c;
   }
 }
@@ -1459,12 +1459,6 @@ void cast_f16_f32(pfhip_backend* b, const uint16_t* s, float* d, size_t n) {
   hipLaunchKernelGGL(k_cast_f16_f32, dim3(grid1d(n)), dim3(256), 0, b->stream, s, d, n);
   PF_HIP(hipGetLastError());
 }
-void cast_f16_f32_ieee(pfhip_backend* b, const uint16_t* s, float* d, size_t n) {
-  if (!n) return;
-  ProfScope ps(b, "cast_logits_f32");
-  hipLaunchKernelGGL(k_cast_f16_f32_ieee, dim3(grid1d(n)), dim3(256), 0, b->stream, s, d, n);
-  PF_HIP(hipGetLastError());
-}
 void cast_f32_f16_scaled(pfhip_backend* b, const float* s, uint16_t* d, size_t n, float scale) {
   if (!n) return;
   ProfScope ps(b, "cast_f32_to_fp16_scaled");
@@ -1552,9 +1546,22 @@ void moe_route(pfhip_backend* b, const int32_t* idx, int T, int K, int E, const 
     PF_HIP(hipGetLastError());
     return;
   }
+  // Count, then the plan from the counts: two kernels, 9.6 us at 2048 tokens
+  // against 16.1 for count, scan and scatter. Every block of the second sums all
+  // counts (quadratic in T), so those three stay from 65536 tokens on.
+  if (T < 65536) {
+    {
+      ProfScope ps(b, "moe_count");
+      hipLaunchKernelGGL(k_moe_count<SMALL_RBLK>, dim3((T + SMALL_RBLK - 1) / SMALL_RBLK), dim3(SMALL_RBLK), 0,
+                         b->stream, idx, m.tile_counts, T, K, E);
+      PF_HIP(hipGetLastError());
+    }
+    moe_route_counts(b, idx, m.tile_counts, SMALL_RBLK, T, K, E, m);
+    return;
+  }
   {
     ProfScope ps(b, "moe_count");
-    hipLaunchKernelGGL(k_moe_count, dim3(nblk), dim3(RBLK), 0, b->stream, idx, m.counts, T, K, E);
+    hipLaunchKernelGGL(k_moe_count<RBLK>, dim3(nblk), dim3(RBLK), 0, b->stream, idx, m.counts, T, K, E);
     PF_HIP(hipGetLastError());
   }
   {
