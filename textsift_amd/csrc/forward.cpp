@@ -687,8 +687,8 @@ static void stage_need(pfhip_model* m, HostStage& st, size_t n) {
     st = HostStage{};
   }
   PF_HIP(hipHostMalloc(&st.host, want, hipHostMallocDefault));
-  st.size = want;
   PF_HIP(hipHostGetDevicePointer(&st.dev, st.host, 0));
+  st.size = want;
 }
 
 // pfhip_model_forward's staging. Up to STAGE_MAX bytes of logits go through
