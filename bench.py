@@ -48,6 +48,7 @@ KERNEL_LABELS = [
     ("gemm_qkv_rope", ("k_gemm_w4<", "(pf::Epi)2, false")),
     ("gemm_o_add_rmsnorm", ("k_gemm_w4_rownorm",)),
     ("gemm_o", ("k_gemm_w4<4, 128", "(pf::Epi)0, false")),
+    ("gemm_o", ("k_gemm_w4<2, 64", "(pf::Epi)0, false")),
     ("gemm_o", ("k_gemm_w4<1, 16", "(pf::Epi)0, false, 4, 7,")),      # all-K small tile, K = 896
     ("gemm_router", ("k_gemm_w4<2, ", "(pf::Epi)5, false")),
     ("gemm_router", ("k_gemm_w4<2, ", "(pf::Epi)1, false")),
