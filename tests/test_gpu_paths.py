@@ -89,6 +89,32 @@ def test_matmul_int4_chunked(be, T, N, K, zp, x_f32):
     assert err < 4 * 2.0 ** -23 * np.sqrt(K / 32) + 2.0 ** -22
 
 
+def test_matmul_int4_grid_limit():
+    """A product whose 32 x 64 tiles would be 2^24 workgroups of 256 threads
+    (a launch holds fewer than 2^32 threads) runs on the larger tiles: 64 GiB
+    of output, checked at the first, middle and last rows against a small call."""
+    T, N, K, n = (1 << 24) - 1, 2052, 128, 40
+    w = synth.qweight(1350, N, K)
+    x = synth.normal(1351, 3 * n * K).astype(np.float32).reshape(3, n, K)
+    be = _native.Backend(0)  # its own: the scratch planes (8 GiB) go with it
+    try:
+        wb = [be.buffer(w[k]) for k in ("int4", "scales", "zp", "bias")]
+        xb, out = be.buffer(nbytes=T * K * 4), be.buffer(nbytes=T * N * 2)
+        be.dispatch("zero_f32", [xb], u32s(T * K, 0, 0, 0))
+        at = [0, T // 2, T - n]
+        for r, v in zip(at, x):
+            xb.write(v, r * K * 4)
+        be.dispatch("matmul_int4_f32_f16", [xb] + wb + [out], u32s(T, N, K, 0))
+        for r, v in zip(at, x):
+            ref = run(be, "matmul_int4_f32_f16", [v] + [w[k] for k in ("int4", "scales", "zp", "bias")], n * N * 2,
+                      u32s(n, N, K, 0)).view(np.uint16)
+            assert np.array_equal(out.read(np.uint16, n * N, r * N * 2), ref), r
+        for b in wb + [xb, out]:
+            b.release()
+    finally:
+        be.close()
+
+
 @pytest.mark.parametrize("T", [100, 1025, 2049])
 def test_moe_layer_split_expert_tiles(be, T):
     """The split MoE layer on the 16-, 32- and 64-row expert tiles (3, 32 and

@@ -272,7 +272,7 @@ void launch(pfhip_backend* b, const GemmArgs& a, const char* name) {
   const int t_tiles = GROUPED ? a.max_tiles : (a.M + BT - 1) / BT;
   const long grid = (long)n_tiles * t_tiles;
   if (grid == 0) return;
-  PF_CHECK(grid < (1L << 31), "gemm_int4: grid too large");
+  PF_CHECK(grid <= MAX_GRID_256, "gemm_int4: grid too large");
   ProfScope ps(b, name);
   hipLaunchKernelGGL((k_gemm_int4<BT, SPLIT, EPI, GROUPED>), dim3((unsigned)grid), dim3(256), 0, b->stream, a);
   PF_HIP(hipGetLastError());
@@ -587,32 +587,34 @@ __global__ __launch_bounds__(256, 2) void k_gemm_int4_k128(GemmArgs p) {
   }
 }
 
+// false: more workgroups than a launch holds (the larger tiles of the kernel above may still fit)
 template <int WF, int BT, bool SPLIT, Epi EPI, bool GROUPED, int CT>
-void launch_k128_ct(pfhip_backend* b, const GemmArgs& a, const char* name) {
+bool launch_k128_ct(pfhip_backend* b, const GemmArgs& a, const char* name) {
   constexpr int BNW = 64 * WF;
   const int t_tiles = GROUPED ? a.max_tiles : (a.M + BT - 1) / BT;
   const long grid = (long)((a.N + BNW - 1) / BNW) * t_tiles;
-  if (grid == 0) return;
-  PF_CHECK(grid < (1L << 31), "gemm_int4: grid too large");
+  if (grid == 0) return true;
+  if (grid > MAX_GRID_256) return false;
   const size_t lds = (size_t)2 * (SPLIT ? 2 : 1) * BT * KC * 2 + (size_t)2 * 4 * BNW * 4;
   const auto kern = &k_gemm_int4_k128<WF, BT, SPLIT, EPI, GROUPED, CT>;
   allow_lds(reinterpret_cast<const void*>(kern), lds);
   ProfScope ps(b, name);
   hipLaunchKernelGGL(kern, dim3((unsigned)grid), dim3(256), lds, b->stream, a);
   PF_HIP(hipGetLastError());
+  return true;
 }
 
 // K = 640 (the model's width) is built with its chunk count, others loop.
 template <int WF, int BT, bool SPLIT, Epi EPI, bool GROUPED>
-void launch_k128(pfhip_backend* b, const GemmArgs& a, const char* name) {
+bool launch_k128(pfhip_backend* b, const GemmArgs& a, const char* name) {
   if (a.K == 5 * KC) return launch_k128_ct<WF, BT, SPLIT, EPI, GROUPED, 5>(b, a, name);
   if constexpr (!GROUPED && !SPLIT && EPI == Epi::F16)
     if (a.K == 7 * KC) return launch_k128_ct<WF, BT, SPLIT, EPI, GROUPED, 7>(b, a, name);
-  launch_k128_ct<WF, BT, SPLIT, EPI, GROUPED, 0>(b, a, name);
+  return launch_k128_ct<WF, BT, SPLIT, EPI, GROUPED, 0>(b, a, name);
 }
 
 // The tiles below, for the forms that the split forward and the named
-// products use; false: not built (the kernel above takes them).
+// products use; false: not built, or too many workgroups (the kernel above takes them).
 // Dense: 32 tokens x 64 columns at every size (2048 x 1152 x 640, RoPE
 // epilogue: 21.7 us, against 24.4 with 64 x 64 and 34.7 with 64 x 128), but 64
 // tokens from 4096 rows for one fp16 plane (O projection of 8192 rows: 24.3
@@ -626,14 +628,10 @@ bool dispatch_k128(pfhip_backend* b, const GemmArgs& a, bool split, Epi epi, boo
     auto tile = [&](auto wf, auto bt) {
       constexpr int WF = decltype(wf)::value, BT = decltype(bt)::value;
       if (epi == Epi::SWIGLU_SPLIT) {
-        if (split) launch_k128<WF, BT, true, Epi::SWIGLU_SPLIT, true>(b, a, name);
-        else launch_k128<WF, BT, false, Epi::SWIGLU_SPLIT, true>(b, a, name);
-        return true;
+        if (split) return launch_k128<WF, BT, true, Epi::SWIGLU_SPLIT, true>(b, a, name);
+        return launch_k128<WF, BT, false, Epi::SWIGLU_SPLIT, true>(b, a, name);
       }
-      if (epi == Epi::F32 && split) {
-        launch_k128<WF, BT, true, Epi::F32, true>(b, a, name);
-        return true;
-      }
+      if (epi == Epi::F32 && split) return launch_k128<WF, BT, true, Epi::F32, true>(b, a, name);
       return false;
     };
     using I1 = std::integral_constant<int, 1>;
@@ -645,19 +643,15 @@ bool dispatch_k128(pfhip_backend* b, const GemmArgs& a, bool split, Epi epi, boo
   }
   switch (epi) {
     case Epi::F16:
-      if (split) launch_k128<1, 32, true, Epi::F16, false>(b, a, name);
-      else if (a.M >= 4096) launch_k128<1, 64, false, Epi::F16, false>(b, a, name);
-      else launch_k128<1, 32, false, Epi::F16, false>(b, a, name);
-      return true;
+      if (split) return launch_k128<1, 32, true, Epi::F16, false>(b, a, name);
+      if (a.M >= 4096) return launch_k128<1, 64, false, Epi::F16, false>(b, a, name);
+      return launch_k128<1, 32, false, Epi::F16, false>(b, a, name);
     case Epi::F32:
-      if (split) launch_k128<1, 32, true, Epi::F32, false>(b, a, name);
-      else if (a.M >= 4096) launch_k128<1, 64, false, Epi::F32, false>(b, a, name);
-      else launch_k128<1, 32, false, Epi::F32, false>(b, a, name);
-      return true;
+      if (split) return launch_k128<1, 32, true, Epi::F32, false>(b, a, name);
+      if (a.M >= 4096) return launch_k128<1, 64, false, Epi::F32, false>(b, a, name);
+      return launch_k128<1, 32, false, Epi::F32, false>(b, a, name);
     case Epi::ROPE_F16:
-      if (!split) return false;
-      launch_k128<1, 32, true, Epi::ROPE_F16, false>(b, a, name);
-      return true;
+      return split && launch_k128<1, 32, true, Epi::ROPE_F16, false>(b, a, name);
     default: return false;
   }
 }

@@ -871,7 +871,8 @@ void launch(pfhip_backend* b, const GemmArgs& a, const char* name) {
   const int t_tiles = GROUPED ? a.max_tiles : (a.M + BT - 1) / BT;
   const long grid = (long)n_tiles * t_tiles;
   if (grid == 0) return;
-  PF_CHECK(grid < (1L << 31), "gemm_w4: grid too large");
+  static_assert(NW <= 4, "MAX_GRID_256 is for workgroups of at most 256 threads");
+  PF_CHECK(grid <= MAX_GRID_256, "gemm_w4: grid too large");
   PF_CHECK(CT == 0 || a.K == CT * KC, "gemm_w4: K does not match the tile's compile-time chunk count");
   // activation buffers: two (double buffering) or all CT chunks, plus the
   // RoPE table's plane when every chunk buffer is taken

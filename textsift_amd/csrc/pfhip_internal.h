@@ -95,6 +95,10 @@ enum class XKind { F16, SPLIT };
 // top-4 + softmax of each output row into topk_idx / topk_w.
 enum class Epi { F16, F32, ROPE_F16, SWIGLU_SPLIT, SWIGLU_F16, F32_TOPK };
 
+// Workgroups of 256 threads in one launch: a grid counts threads in 32 bits,
+// and one past them runs only in part, without an error.
+constexpr long MAX_GRID_256 = (1L << 24) - 1;
+
 struct GemmArgs {
   const void* x = nullptr;       // activations [rows][K] fp16 (the hi plane in SPLIT mode)
   const uint16_t* x_lo = nullptr;  // SPLIT: the lo plane, same row stride
