@@ -145,6 +145,40 @@ def test_moe_layer_split_expert_tiles(be, T):
     assert err < 2.0 ** -11
 
 
+def test_moe_layer_split_matrix_of_2_gib(be):
+    """An expert weight of 2^31 bytes is beyond the K % 128 == 0 kernel's
+    buffer descriptor: the other kernel runs the 16- and 32-row plans too. A
+    token's output depends on its row alone, so every plan tile gives the bits of the 64-row one."""
+    D, E, K, F = 1024, 1, 1, 1 << 21
+    rng = np.random.default_rng(1450)
+
+    def weight(rows, cols, scale):
+        return [np.frombuffer(rng.bytes(rows * cols // 2), np.uint8),
+                synth.to_fp16_bits(np.full(rows * cols // 32, scale)),
+                np.full(rows * cols // 64, 0x88, np.uint8), np.zeros(rows, np.uint16)]
+
+    T = 80
+    x = synth.to_fp16_bits(synth.normal(1451, T * D)).reshape(T, D)
+    none = np.zeros(16, np.uint8)
+    fixed = [be.buffer(a) for a in [synth.to_fp16_bits(synth.normal(1452, D * E)), none, none, np.zeros(8, np.uint16)] +
+             weight(2 * F, D, 2.0 ** -7) + weight(D, F, 2.0 ** -10)]
+    got = {}
+    try:
+        for n in (T, 40, 20):
+            bufs = [be.buffer(x[:n])] + [be.buffer(nbytes=b) for b in (n * D * 2, n * K * 4, n * K * 4)]
+            be.dispatch("moe_ffn", bufs[:1] + fixed + bufs[1:], u32s(n, D, E, K, F, 0, 0, 0))
+            got[n] = bufs[1].read(np.uint16).reshape(n, D)
+            for b in bufs:
+                b.release()
+    finally:
+        for b in fixed:
+            b.release()
+    y = f16(got[T])
+    assert np.all(np.isfinite(y)) and np.mean(y != 0) > 0.99
+    for n in (40, 20):
+        assert np.array_equal(got[n], got[T][:n]), n
+
+
 @pytest.mark.parametrize("scale", [1.0, 2.0 ** -14, 2.0 ** -24])
 def test_fp16_narrowing_below_normal(be, scale):
     """fp16 narrowing with round-half-up below 2^-14: values around every

@@ -47,9 +47,9 @@ namespace pf {
 // rounds of 2 workgroups per CU, against 4 per CU of the smaller tiles.
 ExpertTile expert_tile(int M, int topk, int experts, bool fp16, int D, int F) {
   const int per_expert = (int)((long)M * topk / experts);
-  // split numerics, K % 128 == 0: gemm_int4's tiles of 16, 32 and 64 rows (measured there)
-  if (!fp16 && D % 128 == 0 && F % 128 == 0) return {per_expert < 32 ? 16 : per_expert < 64 ? 32 : 64, 1};
-  if (!fp16) return {per_expert >= 256 ? 128 : 64, 5};
+  // split numerics (gemm_int4, which takes no wf), K % 128 == 0: tiles of 16, 32 and 64 rows (measured there)
+  if (!fp16 && D % 128 == 0 && F % 128 == 0) return {per_expert < 32 ? 16 : per_expert < 64 ? 32 : 64, 0};
+  if (!fp16) return {per_expert >= 256 ? 128 : 64, 0};
   if (per_expert >= 320) return {128, 4};
   const auto small_k = [](int k) { return k == 640 || k == 896; };
   if (small_k(D) && small_k(F) && per_expert < 24) return {16, 1};

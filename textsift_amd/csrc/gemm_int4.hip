@@ -700,7 +700,9 @@ void gemm_int4(pfhip_backend* b, const GemmArgs& a, XKind xk, Epi epi, bool grou
                       ((a.wz_gs & 1) | (a.ws_gs & 1)) == 0 && (long)a.N * a.K / 2 < (1L << 31);
     if (k128 && dispatch_k128(b, a, split, epi, grouped, tile_t, prof_name)) return;
   }
-  if (tile_t == 64) {
+  // The kernel above takes what that one does not (its descriptors hold one matrix below 2^31 bytes):
+  // any plan of up to 64 rows per tile on 64-row tiles, whose rows come from the tile list.
+  if (tile_t == 64 || (grouped && (tile_t == 16 || tile_t == 32))) {
     if (split) {
       if (grouped) dispatch_epi<64, true, true>(b, a, epi, prof_name);
       else dispatch_epi<64, true, false>(b, a, epi, prof_name);
@@ -709,7 +711,7 @@ void gemm_int4(pfhip_backend* b, const GemmArgs& a, XKind xk, Epi epi, bool grou
       else dispatch_epi<64, false, false>(b, a, epi, prof_name);
     }
   } else {
-    PF_CHECK(tile_t == 128, "gemm_int4: tile_t must be 64 or 128");
+    PF_CHECK(tile_t == 128, "gemm_int4: tile_t must be 64 or 128 (grouped: 16, 32, 64 or 128)");
     if (split) {
       if (grouped) dispatch_epi<128, true, true>(b, a, epi, prof_name);
       else dispatch_epi<128, true, false>(b, a, epi, prof_name);
