@@ -139,7 +139,11 @@ int pfhip_model_finalize(pfhip_model* m, char* err, size_t err_cap);
 
 /* Host in / host out (WasmBackend.forward contract, browser/backends/wasm.ts:728-805):
  * ids int32 [batch*seq_len], mask uint8 [batch*seq_len] or NULL (all ones),
- * logits float32 [batch*seq_len*classes] = fp16-rounded logits widened. */
+ * logits float32 [batch*seq_len*classes] = fp16-rounded logits widened.
+ * Calls of up to 32 MiB of logits go through pinned host memory that stays with
+ * the model until pfhip_model_destroy, in powers of two from 64 KiB: at most
+ * 32 MiB for the logits, four bytes a token for the ids and one for the mask.
+ * Where it cannot be had, and above, pageable memory is copied: same results. */
 int pfhip_model_forward(pfhip_model* m, const int32_t* ids, const uint8_t* mask, uint32_t batch, uint32_t seq_len,
                         float* logits, char* err, size_t err_cap);
 /* Device in / device out: same, with inputs already resident in HBM.

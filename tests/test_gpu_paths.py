@@ -1,11 +1,14 @@
 """GPU tests of kernel variants and dispatch rules at the sizes where they
 change: key-mask bits of the attention tiles and its split of the query heads."""
 import struct
+import subprocess
+import sys
 
 import numpy as np
 import pytest
 
 import oracle
+from conftest import ROOT
 from parity_util import rel_err_norm
 from textsift_amd import _native, synth
 
@@ -276,6 +279,72 @@ def test_host_forward_staging(be):
                 m.forward(np.zeros(B * T, np.int32), None, B, T)
     finally:
         m.close()
+
+
+# hipHostMalloc in front of the runtime's: the first `pass` calls go through, later ones report no memory
+# (and record an error, which hipGetDevice(NULL) does here)
+NO_PINNED = """
+#include <dlfcn.h>
+#include <stddef.h>
+extern int hipGetDevice(int*);
+int pass;
+int hipHostMalloc(void** p, size_t n, unsigned flags) {
+  static int (*real)(void**, size_t, unsigned);
+  if (!real) {
+    Dl_info info;
+    dladdr((void*)&hipGetDevice, &info);
+    real = (int (*)(void**, size_t, unsigned))dlsym(dlopen(info.dli_fname, RTLD_NOW), "hipHostMalloc");
+  }
+  if (pass-- > 0) return real(p, n, flags);
+  hipGetDevice(NULL);
+  return 2;
+}
+"""
+
+NO_PINNED_RUN = """
+import ctypes, sys
+import numpy as np
+stub = ctypes.CDLL(sys.argv[1], mode=ctypes.RTLD_GLOBAL)
+passes = ctypes.c_int.in_dll(stub, "pass")
+from textsift_amd import _native, synth
+from textsift_amd.config import PF_CONFIG
+V, C = 512, PF_CONFIG.num_classes
+w = synth.make_model_weights(PF_CONFIG, seed=5, num_layers=1, num_experts=8, vocab_size=V)
+be = _native.Backend(0)
+for allowed in (0, 1, 2):  # none, the ids', the ids' and the logits' memory
+    m = _native.Model(be, PF_CONFIG, num_layers=1, num_experts=8, vocab_size=V)
+    for k, v in w.items():
+        m.set_weight(k, v)
+    m.finalize()
+    passes.value = allowed
+    for i, (B, T, masked) in enumerate([(1, 5, True), (1, 5, True), (1, 5, True), (2, 700, True), (1, 600, False)]):
+        n = B * T
+        ids = synth.token_ids(1900 + i, n, V)
+        mask = (synth.uniform(1950 + i, n) > 0.3).astype(np.uint8) if masked else np.ones(n, np.uint8)
+        got = m.forward(ids, mask, B, T)
+        ib, mb, lb = be.buffer(ids), be.buffer(mask), be.buffer(nbytes=n * C * 4)
+        m.forward_device(ib, mb if masked else None, B, T, lb)
+        assert np.array_equal(got.view(np.uint32), lb.read(np.uint32)), (allowed, B, T)
+        for b in (ib, mb, lb):
+            b.release()
+    assert passes.value < 0  # pinned memory was refused
+    m.close()
+be.close()
+print("equal without pinned memory")
+"""
+
+
+def test_host_forward_without_pinned_memory(tmp_path):
+    """Where pinned memory cannot be had (all of it, or only some of the three
+    blocks) pfhip_model_forward copies pageable memory and gives the
+    device-resident forward's bits."""
+    src, so = tmp_path / "no_pinned.c", tmp_path / "no_pinned.so"
+    src.write_text(NO_PINNED)
+    subprocess.run(["gcc", "-shared", "-fPIC", "-D_GNU_SOURCE", str(src), "-o", str(so), "-L/opt/rocm/lib",
+                    "-lamdhip64", "-ldl", "-Wl,-rpath,/opt/rocm/lib"], check=True)
+    r = subprocess.run([sys.executable, "-c", NO_PINNED_RUN, str(so)], cwd=ROOT, capture_output=True, text=True,
+                       timeout=100)
+    assert r.returncode == 0 and "equal without pinned memory" in r.stdout, r.stdout + r.stderr
 
 
 # ---------------------------------------------------------------- routing plan

@@ -675,27 +675,39 @@ static void enqueue_forward(pfhip_model* m, const int32_t* idp, const uint8_t* m
 }
 
 // Grows st to at least n bytes (powers of two from 64 KiB: pinning is slow).
-// Captured forwards may name the old memory: they go with it.
-static void stage_need(pfhip_model* m, HostStage& st, size_t n) {
-  if (st.size >= n) return;
+// Captured forwards may name the old memory: they go with it. False, with
+// nothing held, where there is no pinned memory of that size.
+static bool stage_need(pfhip_model* m, HostStage& st, size_t n) {
+  if (st.size >= n) return true;
   size_t want = 64 << 10;
   while (want < n) want <<= 1;
-  clear_graphs(m);
   if (st.host) {
+    clear_graphs(m);
     PF_HIP(hipStreamSynchronize(m->b->stream));
     hipHostFree(st.host);
     st = HostStage{};
   }
-  PF_HIP(hipHostMalloc(&st.host, want, hipHostMallocDefault));
-  PF_HIP(hipHostGetDevicePointer(&st.dev, st.host, 0));
+  if (hipHostMalloc(&st.host, want, hipHostMallocDefault) != hipSuccess) {
+    st = HostStage{};
+    (void)hipGetLastError();  // not a launch's error
+    return false;
+  }
+  if (hipHostGetDevicePointer(&st.dev, st.host, 0) != hipSuccess) {
+    hipHostFree(st.host);
+    st = HostStage{};
+    (void)hipGetLastError();
+    return false;
+  }
   st.size = want;
+  return true;
 }
 
 // pfhip_model_forward's staging. Up to STAGE_MAX bytes of logits go through
 // pinned memory kept with the model: the embedding kernel reads the ids there, the
 // logits are written there (by the classifier itself up to STAGE_DIRECT bytes,
 // whose scattered stores a copy kernel's whole lines beat above), and the
-// host waits once. Larger batches copy pageable memory, with a wait per copy.
+// host waits once. Larger batches, and calls for which pinned memory cannot be
+// had, copy pageable memory, with a wait per copy.
 // 8 layers of 1 x 25 tokens: 501 -> 463 us; one layer of 12 x 1000 masked tokens: 473 -> 432.
 constexpr size_t STAGE_MAX = (size_t)32 << 20;
 constexpr size_t STAGE_DIRECT = (size_t)64 << 10;
@@ -947,7 +959,10 @@ int pfhip_model_forward(pfhip_model* m, const int32_t* ids, const uint8_t* mask,
         }
     const size_t lbytes = M * m->cfg.classes * 4;
     if (use_mask) ensure(m->mask_buf, M);
-    if (lbytes > STAGE_MAX) {
+    const bool staged = lbytes <= STAGE_MAX && stage_need(m, m->ids_st, M * 4) &&
+                        stage_need(m, m->logits_st, al256(lbytes)) &&
+                        (!use_mask || stage_need(m, m->mask_st, al256(M)));
+    if (!staged) {
       ensure(m->ids_buf, M * 4);
       ensure(m->logits_buf, lbytes);
       PF_CHECK(pfhip_write_buffer(m->b, m->ids_buf, 0, ids, M * 4, e2, sizeof e2) == 0, e2);
@@ -960,11 +975,8 @@ int pfhip_model_forward(pfhip_model* m, const int32_t* ids, const uint8_t* mask,
     }
     const bool direct = lbytes <= STAGE_DIRECT;
     if (!direct) ensure(m->logits_buf, lbytes);
-    stage_need(m, m->ids_st, M * 4);
-    stage_need(m, m->logits_st, al256(lbytes));
     memcpy(m->ids_st.host, ids, M * 4);
     if (use_mask) {  // read by every layer's attention: copied to the device
-      stage_need(m, m->mask_st, al256(M));
       memcpy(m->mask_st.host, mask, M);
       copy16(m->b, m->mask_st.dev, m->mask_buf->ptr, (M + 15) & ~(size_t)15);
     }
