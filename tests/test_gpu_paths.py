@@ -44,13 +44,15 @@ def run(be, name, inputs, out_bytes, pushb):
 # ---------------------------------------------------------------- attention
 
 @pytest.mark.parametrize("hw_exp", [0, 1], ids=["wasm-exp", "hw-exp"])
-@pytest.mark.parametrize("T,W", [(1, 128), (45, 128), (161, 128), (1000, 128), (130, 8), (12900, 128)])
+@pytest.mark.parametrize("T,W", [(1, 128), (45, 128), (161, 128), (1000, 128), (130, 8), (12900, 128), (16500, 128),
+                                 (9600, 16), (32000, 16), (24000, 32), (8320, 64)])
 def test_attention_key_mask(be, T, W, hw_exp):
     """Masked runs that empty whole 32-key chunks, scattered masked keys and
     mask bytes other than 0 and 1, against the oracle with the tolerances of
     the unmasked test: fp16 outputs (2^-11) of the same arithmetic, and in the
-    hardware-exp form one more fp16 rounding of the weights. 12900 tokens make
-    more workgroups than CUs (one workgroup per KV head), the others split the heads."""
+    hardware-exp form one more fp16 rounding of the weights. Every tile (windows 8,
+    16, 32, 64 and 128) and splits of the 7 heads into 1, 2 and more, with
+    fewer workgroups than CUs (up to 12900 tokens at window 128) and more (16500)."""
     Hq, Hkv, hd = 14, 2, 64
     q = synth.to_fp16_bits(synth.normal(900 + T, T * Hq * hd, 0, 0.35))
     k = synth.to_fp16_bits(synth.normal(901 + T, T * Hkv * hd, 0, 0.35))

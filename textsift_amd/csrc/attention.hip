@@ -8,11 +8,12 @@
 // 4-lane vector part and libm exp for its scalar tail; p_i = e_i / sum(e, sink);
 // out = fp16(sum_i p_i v_i). Masked keys score -inf.
 //
-// Mapping to CDNA4 (one workgroup = 4 waves = 64 query tokens of one
-// sequence and one KV head, all Hq/Hkv query heads of that group):
-//  * The workgroup stages its union of keys (64 + 2W rows) once in LDS:
-//    K row-major, V transposed (V^T[dim][key]); every query head of the
-//    group reuses them.
+// Mapping to CDNA4 (one workgroup = 8 waves = 128 query tokens of one
+// sequence and one KV head, 4 waves and 64 tokens for windows up to 40, and
+// an even share of the Hq/Hkv query heads of that group):
+//  * The workgroup stages its union of keys (128 or 64 + 2W rows) once in LDS:
+//    K row-major, V transposed (V^T[dim][key]); each of its query heads
+//    reuses them.
 //  * S^T = K . Q^T on v_mfma_f32_16x16x32_f16 leaves each lane holding 4
 //    consecutive keys of one query; two such 16-key tiles are exactly the
 //    B-operand fragment of the P.V MFMA (O^T = V^T . P^T), so P never
@@ -623,19 +624,33 @@ __global__ __launch_bounds__(64 * NW) void k_banded_attention_hw(AttnArgs a) {
   }
 }
 
-// Workgroups per KV head: its G query heads are split evenly over them (each
-// stages the K/V rows for its own heads). The launch takes rounds of
-// `resident` workgroups at a time, each as long as its largest share of heads
-// plus the staging, which costs about one head (34 us for 7 heads, 23 us for
-// 4): the split with the least rounds x (heads + 1), the coarsest on a tie.
-// (The fewest workgroups that give every CU one, the earlier rule, took two
-// rounds of 4 heads at 12 x 1000 tokens, where one round of 7 fits: 9 us more.)
-int attn_head_groups(long wgs, int G, long resident) {
+// Workgroups per KV head: its G query heads are split evenly over g of them
+// (each stages the K/V rows for its own heads). A CU runs n = ceil(wgs g /
+// CUs) of them, each as long as its heads (the larger share while n <= 2, the
+// mean when more even out) plus the staging; a CU that could hold several at
+// once is far from busy with one, which takes `lone` times as long as its share
+// of a full CU. The g of least cost, the coarsest on a tie. stage (in heads) and
+// lone are fitted to 126 sizes (14 query and 2 KV heads, windows 8 to 128, 8
+// to 2100 workgroups, g = 1, 2, 3, 4 and 7): at window 128 the choice is within 2 % of
+// the fastest of these g, elsewhere within 10 %. us at g = 1 / 2 / 3 / 4 / 7:
+//   window 128, hardware exp:  128 workgroups 28.8 / 20.9 / 27.6 / 24.8 / 33.6
+//                              160: 29.9 / 34.0 / 30.9 / 32.5 / 41.5
+//                              260: 54.8 / 49.4 / 52.8 / 52.8 / 67.7
+//                              520: 84.9 / 88.8 / 95.3 / 101.9 / 126.3
+//   window 128, WASM exp:      160: 77.9 / 75.8 / 66.0 / 63.6 / 66.9
+//                              260: 136.8 / 104.8 / 101.1 / 93.6 / 107.0
+//   window 16, hardware exp:   300: 17.6 / 15.8 / 16.6 / 18.5 / 21.1
+//                              1000: 29.8 / 35.2 / 42.3 / 43.2 / 55.4
+// (An earlier rule counted whole rounds of resident workgroups, with one head
+// for the staging; it took g = 2 in the last of these.)
+int attn_head_groups(long wgs, int G, long cus, double stage, double lone) {
   int best = 1;
-  long cost = -1;
+  double cost = 0.0;
   for (int g = 1; g <= G; ++g) {
-    const long c = ((wgs * g + resident - 1) / resident) * ((G + g - 1) / g + 1);
-    if (cost < 0 || c < cost) {
+    const long n = (wgs * g + cus - 1) / cus;
+    const int most = (G + g - 1) / g;
+    const double c = std::max(lone * (most + stage), n * ((n <= 2 ? (double)most : (double)G / g) + stage));
+    if (g == 1 || c < cost) {
       best = g;
       cost = c;
     }
@@ -644,12 +659,11 @@ int attn_head_groups(long wgs, int G, long resident) {
 }
 
 template <typename Kern>
-void launch_kernel(pfhip_backend* b, const AttnArgs& a, Kern* kern, size_t lds, int qb, int nt) {
+void launch_kernel(pfhip_backend* b, const AttnArgs& a, Kern* kern, size_t lds, int qb, int nt, double lone) {
   allow_lds(reinterpret_cast<const void*>(kern), lds);
   AttnArgs g = a;
   const long wgs = (long)((a.T + qb - 1) / qb) * a.Hkv * a.B;
-  // resident workgroups: the 8-wave tiles hold 2 waves per SIMD (registers), the 4-wave ones 3
-  g.head_groups = attn_head_groups(wgs, a.Hq / a.Hkv, (long)b->num_cus * (nt > 256 ? 1 : 3));
+  g.head_groups = attn_head_groups(wgs, a.Hq / a.Hkv, b->num_cus, a.hw_exp ? 2.5 : 0.5, lone);
   dim3 grid((a.T + qb - 1) / qb, a.Hkv * g.head_groups, a.B);
   ProfScope ps(b, "banded_attention");
   hipLaunchKernelGGL(kern, grid, dim3(nt), lds, b->stream, g);
@@ -660,12 +674,16 @@ template <int HD, int NCH, int NW>
 void launch_attn(pfhip_backend* b, const AttnArgs& a) {
   constexpr size_t LDS = AttnGeom<HD, NCH, NW>::LDS;
   static_assert(LDS <= 160 * 1024, "attention tile exceeds the LDS");
+  // attn_head_groups' lone: a CU holds 6, 4 or 3 workgroups of the 4-wave tiles of
+  // 1, 2 or 3 chunks and two of the WASM form's 8-wave tile of 5; one of the others (registers)
+  constexpr double LONE = NW == 4 ? (NCH < 3 ? 2.5 : 2.0) : 1.0;
+  constexpr double LONE_WASM = NCH == 5 ? 2.0 : LONE;
   if (a.hw_exp) {
-    if (a.mask) launch_kernel(b, a, &k_banded_attention_hw<HD, NCH, NW, true>, LDS, 16 * NW, 64 * NW);
-    else launch_kernel(b, a, &k_banded_attention_hw<HD, NCH, NW, false>, LDS, 16 * NW, 64 * NW);
+    if (a.mask) launch_kernel(b, a, &k_banded_attention_hw<HD, NCH, NW, true>, LDS, 16 * NW, 64 * NW, LONE);
+    else launch_kernel(b, a, &k_banded_attention_hw<HD, NCH, NW, false>, LDS, 16 * NW, 64 * NW, LONE);
   } else {
-    if (a.mask) launch_kernel(b, a, &k_banded_attention<HD, NCH, NW, true>, LDS, 16 * NW, 64 * NW);
-    else launch_kernel(b, a, &k_banded_attention<HD, NCH, NW, false>, LDS, 16 * NW, 64 * NW);
+    if (a.mask) launch_kernel(b, a, &k_banded_attention<HD, NCH, NW, true>, LDS, 16 * NW, 64 * NW, LONE_WASM);
+    else launch_kernel(b, a, &k_banded_attention<HD, NCH, NW, false>, LDS, 16 * NW, 64 * NW, LONE_WASM);
   }
 }
 
