@@ -209,11 +209,14 @@ def prepared(be, q, rows, K):
     return out + [be.buffer(q["bias"])]
 
 
-@pytest.mark.parametrize("T,N,K", [(704, 1152, 640), (705, 1152, 640), (1280, 640, 896), (1281, 640, 896),
+@pytest.mark.parametrize("T,N,K", [(672, 1152, 640), (673, 1152, 640), (5440, 1152, 640), (5441, 1152, 640),
+                                   (6528, 1152, 640), (6529, 1152, 640), (1216, 640, 896), (1217, 640, 896),
+                                   (704, 1152, 640), (705, 1152, 640), (1280, 640, 896), (1281, 640, 896),
                                    (10240, 1152, 640), (10241, 1152, 640), (10241, 640, 896), (300, 72, 256)])
 def test_matmul_w4_tile_rule(be, T, N, K):
-    """The dense tile the library chooses on each side of every line of its
-    rule gives the bits of the 64 x 64 tile."""
+    """The dense tile the library chooses gives the bits of the 64 x 64 tile: on
+    each side of the first lines of its rule on 256 CUs (16 x 64, 64 x 128, 128 x 256 and
+    back at N = 1152; 16 x 64 to 64 x 128 at K = 896), and at larger and odd sizes."""
     w = prepared(be, synth.qweight(1500 + N, N, K), N, K)
     x, out = be.buffer(synth.to_fp16_bits(synth.normal(1501, T * K))), be.buffer(nbytes=T * N * 2)
     got = []

@@ -56,17 +56,26 @@ ExpertTile expert_tile(int M, int topk, int experts, bool fp16, int D, int F) {
   return {per_expert < 48 ? 32 : 64, 2};
 }
 
-// Tile of a dense fp16-numerics GEMM without a top-k epilogue. 16 x 64 (all
-// of K at once, K = 640 or 896) while 64 x 128 tiles are fewer than 100:
-// 437 x 1152 x 640 5.9 against 7.3 us, 1024 x 1152 x 640 9.2 against 7.2. Then 64 x
-// 128, up to 10240 rows against 128 x 256 (8192 x 1152 x 640 20.9 / 24.2 us, 12000: 27.5 /
-// 25.7), and at any size where 256 columns would be padded by over an eighth (12000 x 640 x 896
-// 22.7 / 30.2 us).
-ExpertTile dense_tile(int M, int N, int K) {
-  const long tiles = (long)((M + 63) / 64) * ((N + 127) / 128);
-  if ((K == 640 || K == 896) && tiles < 100) return {16, 1};
-  const long padded = (long)((N + 255) / 256) * 256;
-  return M > 10240 && 8 * padded <= 9 * (long)N ? ExpertTile{128, 4} : ExpertTile{64, 2};
+// Tile of a dense fp16-numerics GEMM without a top-k epilogue: 16 x 64 (all of
+// K at once, K = 640 or 896), 64 x 128 or 128 x 256, whichever a CU is done with first. Its
+// time goes with n = tiles / CUs, in whole tiles and a part that is linear (memory), and with
+// K: us = launch + K / 640 (whole ceil(n) + linear n), fitted to 41 row
+// counts from 300 to 32768 of twelve (N, K). There the choice is 0.1 % behind the fastest
+// on average and at most 9 % (one of 492: 32768 x 256 x 640, 21.7 against 18.7).
+// us on 16 x 64 / 64 x 128 / 128 x 256:
+//   437 x 1152 x 640  5.9 / 7.3 / -        704 x 1152 x 640   7.4 / 7.1 / 14.5
+//   600 x 1280 x 640  6.6 / 7.1 / 14.5     2048 x 640 x 896  10.9 / 8.6 / 19.0
+//   8192 x 1152 x 640  - / 20.9 / 24.2     10000 x 1280 x 640   - / 28.0 / 25.6
+//   12000 x 1152 x 640 - / 27.5 / 25.7     12000 x 640 x 896    - / 22.7 / 30.2
+//   14000 x 1152 x 640 - / 32.3 / 35.5     20000 x 640 x 1024   - / 42.9 / 35.6
+ExpertTile dense_tile(int cus, int M, int N, int K) {
+  const auto us = [&](int rows, int cols, double launch, double whole, double linear) {
+    const double tiles = (double)((M + rows - 1) / rows) * ((N + cols - 1) / cols);
+    return launch + K / 640.0 * (whole * std::ceil(tiles / cus) + linear * tiles / cus);
+  };
+  const double t16 = us(16, 64, 3.7, 0.77, 0.25), t64 = us(64, 128, 4.3, 2.5, 0.9), t128 = us(128, 256, 7.1, 6.3, 4.0);
+  if ((K == 640 || K == 896) && t16 <= std::min(t64, t128)) return {16, 1};
+  return t128 < t64 ? ExpertTile{128, 4} : ExpertTile{64, 2};
 }
 }  // namespace pf
 
@@ -483,7 +492,7 @@ static void run_forward(pfhip_model* m, const int32_t* ids, const uint8_t* mask,
       a.seq_len = T; a.rope_cols = (Hq + Hkv) * hd;
       if (f16) {
         a.w = reinterpret_cast<const uint8_t*>(L.qkv4.w); a.wsz = L.qkv4.sz;
-        const ExpertTile t = dense_tile(M, NQKV, D);
+        const ExpertTile t = dense_tile(b->num_cus, M, NQKV, D);
         gemm_w4(b, a, XKind::F16, Epi::ROPE_F16, false, t.t, t.wf, "gemm_qkv_rope");
       } else {
         gemm_int4(b, a, XKind::SPLIT, Epi::ROPE_F16, false, 128, "gemm_qkv_rope");
@@ -516,7 +525,7 @@ static void run_forward(pfhip_model* m, const int32_t* ids, const uint8_t* mask,
         if (fused_o) {
           gemm_w4_add_rmsnorm(b, a, h, L.ln_post, s.h2, s.xn_hi, c.eps);
         } else {
-          const ExpertTile t = dense_tile(M, D, Hq * hd);
+          const ExpertTile t = dense_tile(b->num_cus, M, D, Hq * hd);
           gemm_w4(b, a, XKind::F16, Epi::F16, false, t.t, t.wf, "gemm_o");
           if (!norm_in_router) add_rms_norm_f16(b, h, s.o, L.ln_post, s.h2, s.xn_hi, M, D, c.eps);
         }

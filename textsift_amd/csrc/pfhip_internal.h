@@ -174,8 +174,8 @@ struct ExpertTile {
 };
 ExpertTile expert_tile(int M, int topk, int experts, bool fp16, int D, int F);
 // The same for a dense gemm_w4 product of M rows (the forward's QKV and O
-// projections and the matmul_w4 named kernel).
-ExpertTile dense_tile(int M, int N, int K);
+// projections and the matmul_w4 named kernel) on cus CUs.
+ExpertTile dense_tile(int cus, int M, int N, int K);
 
 // Scale-folded int4 GEMM (gemm_w4.hip): weights prepared by w4_prepare;
 // K % 128 == 0. tile_t x wf selects the tile (BT tokens x 64*wf rows):

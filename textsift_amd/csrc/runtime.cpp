@@ -241,7 +241,7 @@ static void moe_ffn_fp16(pfhip_backend* b, const uint16_t* x, const uint16_t* rw
 // chooses it for T rows when tile_t == 0.
 static void matmul_w4_auto(pfhip_backend* b, GemmArgs& a, Epi epi, int tile_t, int wf, const char* name) {
   if (tile_t == 0) {
-    const ExpertTile t = dense_tile(a.M, a.N, a.K);
+    const ExpertTile t = dense_tile(b->num_cus, a.M, a.N, a.K);
     tile_t = t.t;
     wf = t.wf;
   }
