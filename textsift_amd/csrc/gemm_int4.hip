@@ -295,8 +295,8 @@ void launch(pfhip_backend* b, const GemmArgs& a, const char* name) {
 //  * The lane's accumulator rows are 4 lg .. + 3 of a fragment, so the f32
 //    scales of the chunk are kept in LDS as [block][row] and read as one
 //    16-byte vector per fragment and block; each thread converts WF of them per chunk.
-// 2048 x 1152 x 640 with the RoPE epilogue: 51.1 us in the kernel above, 21.7
-// here; the 2048-token layer's gate_up and down 85 / 46 -> 66 / 33 us. Of that
+// 2048 x 1152 x 640 with the RoPE epilogue: 51.2 us in the kernel above, 21.5
+// here; the 2048-token layer's gate_up and down 84 / 46 -> 65 / 32 us. Of that
 // the 16-byte weight loads and their transpose (instead of four 4-byte loads) are
 // a fifth, and the RoPE epilogue's branch-free subnormal path 4 us.
 // Bound: per 16 x 16 x 32 block two MFMAs (32 cycles) and 4 fmaf (16), plus

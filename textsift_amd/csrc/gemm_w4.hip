@@ -1038,9 +1038,10 @@ void gemm_w4(pfhip_backend* b, const GemmArgs& a, XKind xk, Epi epi, bool groupe
                  a.plan_tiles && a.plan_num_tiles && a.plan_tile_t >= 1,
              "gemm_w4: the routing plan is built by the single 16-row router tile (M <= 16), with every plan output");
   if (tile_t == 128 && wf == 4) return dispatch_grouped<4, 128>(b, g, epi, grouped, prof_name);
-  // (64, 5) expert tiles with K = 640 load all five chunks at once (80 KB of
-  // LDS, two workgroups per CU): a tile waits for memory once instead of
-  // once per chunk, which is what bounds these GEMMs at a few hundred tiles
+  // (64, 5): asked for by moe_ffn_w4 and matmul_int4_w4 callers only; expert_tile's
+  // (32, 2) and (64, 2), four workgroups per CU, are faster at every row count
+  // (measured there). Expert tiles with K = 640 load all five chunks at once
+  // (80 KB of LDS, two workgroups per CU).
   if (tile_t == 64 && wf == 5 && grouped && a.K == 5 * KC)
     return dispatch_epi<5, 64, 1, true, 4, 5>(b, g, epi, prof_name);
   if (tile_t == 64 && wf == 5) return dispatch_grouped<5, 64>(b, g, epi, grouped, prof_name);

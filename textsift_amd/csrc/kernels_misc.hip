@@ -613,7 +613,7 @@ __device__ __forceinline__ void moe_write_tiles(const int32_t* tile0, const int3
 // counts[blk][e] = tokens of block blk routed to expert e.
 template <int RB>
 __global__ __launch_bounds__(RB) void k_moe_count(const int32_t* __restrict__ idx, int32_t* __restrict__ counts,
-                                                    int T, int K, int E) {
+                                                  int T, int K, int E) {
   constexpr int BW = RB / 32 + 1;
   __shared__ uint32_t bits[256 * BW];
   const int blk = blockIdx.x;
@@ -790,11 +790,11 @@ __global__ __launch_bounds__(RBLK) void k_moe_scatter(const int32_t* __restrict_
 // and blk_off are not written: nothing else reads them).
 template <int RB>
 __global__ __launch_bounds__(RB) void k_moe_route_small(const int32_t* __restrict__ idx,
-                                                          int32_t* __restrict__ expert_off,
-                                                          int32_t* __restrict__ slot_token,
-                                                          int32_t* __restrict__ slot_of, int32_t* __restrict__ tiles,
-                                                          int32_t* __restrict__ num_tiles, int T, int K, int E,
-                                                          int tile_t) {
+                                                        int32_t* __restrict__ expert_off,
+                                                        int32_t* __restrict__ slot_token,
+                                                        int32_t* __restrict__ slot_of, int32_t* __restrict__ tiles,
+                                                        int32_t* __restrict__ num_tiles, int T, int K, int E,
+                                                        int tile_t) {
   constexpr int BW = RB / 32 + 1;
   __shared__ uint32_t bits[256 * BW];
   __shared__ int32_t off[256], toff[256], wsum[2][RB / 64];
@@ -870,12 +870,12 @@ __global__ __launch_bounds__(RB) void k_moe_route_small(const int32_t* __restric
 // expert_off, the tile list and num_tiles. Same outputs as the three kernels.
 template <int RB>
 __global__ __launch_bounds__(RB) void k_moe_route_counts(const int32_t* __restrict__ idx,
-                                                           const int32_t* __restrict__ counts, int n_ct,
-                                                           int ct_per_blk, int32_t* __restrict__ expert_off,
-                                                           int32_t* __restrict__ slot_token,
-                                                           int32_t* __restrict__ slot_of, int32_t* __restrict__ tiles,
-                                                           int32_t* __restrict__ num_tiles, int T, int K, int E,
-                                                           int tile_t) {
+                                                         const int32_t* __restrict__ counts, int n_ct,
+                                                         int ct_per_blk, int32_t* __restrict__ expert_off,
+                                                         int32_t* __restrict__ slot_token,
+                                                         int32_t* __restrict__ slot_of, int32_t* __restrict__ tiles,
+                                                         int32_t* __restrict__ num_tiles, int T, int K, int E,
+                                                         int tile_t) {
   constexpr int BW = RB / 32 + 1;
   __shared__ uint32_t bits[256 * BW];
   __shared__ int32_t psum[2][4 * RB];  // per (part of the tiles, expert): all tiles, tiles before the block
@@ -1298,7 +1298,8 @@ void copy16(pfhip_backend* b, const void* src, void* dst, size_t bytes) {
            "copy16: 16-byte aligned sizes and pointers");
   if (!bytes) return;
   ProfScope ps(b, "copy16");
-  hipLaunchKernelGGL(k_copy16, dim3((unsigned)std::min<size_t>(4096, (bytes / 16 + 255) / 256)), dim3(256), 0, b->stream, static_cast<const u4_t*>(src),
+  const unsigned grid = (unsigned)std::min<size_t>(4096, (bytes / 16 + 255) / 256);
+  hipLaunchKernelGGL(k_copy16, dim3(grid), dim3(256), 0, b->stream, static_cast<const u4_t*>(src),
                      static_cast<u4_t*>(dst), bytes / 16);
   PF_HIP(hipGetLastError());
 }
