@@ -62,39 +62,45 @@ struct AttnGeom {
   static constexpr size_t KV = (size_t)(ROWS * LDK + HD * LDV) * 2;
   static constexpr size_t LDS = KV + ROWS;  // then the staged rows' key-mask bytes
   static_assert(LDV % 8 == 4, "V^T row stride must be 2 mod 4 dwords");
-  static_assert(KV % 16 == 0 && ROWS <= 64 * NW, "mask bytes: aligned words, one per thread");
+  static_assert(ROWS <= 64 * NW, "mask bytes: one per thread");
 };
 
-// The key mask of a wave's band as bits: bit 8 (c & 3) + 4 kt + r of word
-// c / 4 is set when key row + 32 c + 16 kt + 4 lg + r (a staged row) has a
-// nonzero mask byte. The mask does not depend on the query head, so it is read once
-// per workgroup into LDS (stage_mask) and once per wave into these registers,
-// instead of one global byte load per score and head: 12 sequences of 1000
-// tokens, a quarter of them masked, took 80.8 us with the byte loads and take
-// 34.4 us with the bits, as without a mask.
+// The key mask of a wave's band as bits: bit i of word c is set when staged
+// row + 32 c + i has a nonzero mask byte. The mask does not depend on the query
+// head, so it is read once per workgroup into LDS (stage_mask) and once per
+// wave from there, a byte per lane whose ballot is the bits of two chunks in scalar
+// registers, instead of one global byte load per score and head: 12 sequences of
+// 1000 tokens, a quarter of them masked, 80.5 us with the byte loads and
+// 33.4 with the bits, as without a mask; one masked sequence of 68 tokens 7.7 and
+// 7.6 us, of 2001 14.7 and 10.8 (10.1 without a mask), WASM exponentials 25.3 and 18.9.
 template <int NCH>
 struct KeyBits {
-  static constexpr int NWD = (NCH + 3) / 4;
-  uint32_t w[NWD];
-  __device__ __forceinline__ void load(const uint8_t* mask_lds, int row, int lg) {
+  uint32_t w[NCH];
+  __device__ __forceinline__ void load(const uint8_t* mask_lds, int rows, int row, int lane) {
 #pragma unroll
-    for (int i = 0; i < NWD; ++i) w[i] = 0u;
-#pragma unroll
-    for (int c = 0; c < NCH; ++c)
-#pragma unroll
-      for (int kt = 0; kt < 2; ++kt) {  // 4 bytes of 0 or 1 -> 4 bits
-        const uint32_t b = *reinterpret_cast<const uint32_t*>(mask_lds + row + 32 * c + 16 * kt + 4 * lg);
-        w[c >> 2] |= ((b | b >> 7 | b >> 14 | b >> 21) & 0xFu) << (8 * (c & 3) + 4 * kt);
-      }
+    for (int c = 0; c < NCH; c += 2) {
+      const uint64_t b = __ballot(mask_lds[min(row + 32 * c + lane, rows - 1)] != 0);
+      w[c] = (uint32_t)b;
+      if (c + 1 < NCH) w[c + 1] = (uint32_t)(b >> 32);
+    }
   }
-  __device__ __forceinline__ bool at(int c, int kt, int r) const { return (w[c >> 2] >> (8 * (c & 3) + 4 * kt + r)) & 1u; }
-  // chunks whose every key's bit is v, for the whole wave (bit c)
+  // Called once per head: the lane masks made from the bits are then recomputed where
+  // they are needed, as for the window bounds. (Hoisted out of the head loop, 144 of their
+  // registers spilled, which cost every masked call 1 us: 8.7 at 68 tokens, 11.9 at 2001.)
+  __device__ __forceinline__ void opaque() {
+#pragma unroll
+    for (int c = 0; c < NCH; ++c) asm volatile("" : "+s"(w[c]));
+  }
+  // of the lane group's key 16 kt + 4 lg + r of chunk c
+  __device__ __forceinline__ bool at(int c, int kt, int lg, int r) const {
+    return (w[c] >> (16 * kt + 4 * lg + r)) & 1u;
+  }
+  // chunks whose every key's bit is v (bit c)
   __device__ __forceinline__ uint32_t all(bool v) const {
     uint32_t f = 0u;
 #pragma unroll
-    for (int c = 0; c < NCH; ++c)
-      f |= (uint32_t)__all(((w[c >> 2] >> (8 * (c & 3))) & 0xFFu) == (v ? 0xFFu : 0u)) << c;
-    return __builtin_amdgcn_readfirstlane(f);
+    for (int c = 0; c < NCH; ++c) f |= (uint32_t)(w[c] == (v ? ~0u : 0u)) << c;
+    return f;
   }
 };
 
@@ -221,7 +227,7 @@ __global__ __launch_bounds__(64 * NW) void k_banded_attention(AttnArgs a) {
   [[maybe_unused]] KeyBits<NCH> keys;
   uint32_t key_full = ~0u;  // chunks without a masked key
   if constexpr (MASKED) {
-    keys.load(mask_lds, rb, lg);
+    keys.load(mask_lds, ROWS, rb, lane);
     key_full = keys.all(true);
   }
   const int G = a.Hq / a.Hkv;
@@ -235,6 +241,7 @@ __global__ __launch_bounds__(64 * NW) void k_banded_attention(AttnArgs a) {
     // as dozens of live lane masks (which spill).
     int lo = lo0, hi = hi0, tail = tail0;
     asm volatile("" : "+v"(lo), "+v"(hi), "+v"(tail));
+    if constexpr (MASKED) keys.opaque();
     // Q fragment (B operand): Q[tq][32 dh + 8 lg .. +8]
     h8_t qf[NDH];
 #pragma unroll
@@ -279,7 +286,7 @@ __global__ __launch_bounds__(64 * NW) void k_banded_attention(AttnArgs a) {
             const int off = 32 * c + 16 * kt + 4 * lg + r;
             const bool inwin = (off >= lo) & (off < hi);
             bool valid = inwin;
-            if constexpr (MASKED) valid = valid & keys.at(c, kt, r);
+            if constexpr (MASKED) valid = valid & keys.at(c, kt, lg, r);
             const float sv = valid ? acc[kt][r] * sscale : -INFINITY;
             s[c][kt][r] = inwin ? sv : NAN;
             m = valid ? fmaxf(m, sv) : m;
@@ -439,7 +446,7 @@ __global__ __launch_bounds__(64 * NW) void k_banded_attention_hw(AttnArgs a) {
   [[maybe_unused]] KeyBits<NCH> keys;
   uint32_t key_full = ~0u, key_none = 0u;  // chunks without a masked key, and without any other
   if constexpr (MASKED) {
-    keys.load(mask_lds, rb, lg);
+    keys.load(mask_lds, ROWS, rb, lane);
     key_full = keys.all(true);
     key_none = keys.all(false);
   }
@@ -468,6 +475,7 @@ __global__ __launch_bounds__(64 * NW) void k_banded_attention_hw(AttnArgs a) {
     // opaque per-head copies of the window bounds (see k_banded_attention)
     int lo = lo0, hi = hi0;
     asm volatile("" : "+v"(lo), "+v"(hi));
+    if constexpr (MASKED) keys.opaque();
     const int hn = hh + 1 < h_end ? hq + 1 : hq;
     const float sink_n = load_sink(hn);  // issued before the Q loads: waiting for it leaves them in flight
     h8_t qn[NDH];
@@ -513,7 +521,7 @@ __global__ __launch_bounds__(64 * NW) void k_banded_attention_hw(AttnArgs a) {
             for (int r = 0; r < 4; ++r) {
               const int off = 32 * c + 16 * kt + 4 * lg + r;
               bool valid = (off >= lo) & (off < hi);
-              if constexpr (MASKED) valid = valid & keys.at(c, kt, r);
+              if constexpr (MASKED) valid = valid & keys.at(c, kt, lg, r);
               s[c][kt][r] = valid ? s[c][kt][r] : -INFINITY;
             }
         }
