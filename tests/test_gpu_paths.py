@@ -228,7 +228,7 @@ def test_matmul_w4_tile_rule(be, T, N, K):
     assert np.array_equal(got[0], got[1])
 
 
-@pytest.mark.parametrize("T", [767, 768, 1535, 1536, 10240])
+@pytest.mark.parametrize("T", [767, 768, 1535, 1536, 10239, 10240])
 def test_moe_expert_tile_rule(be, T):
     """The expert tile on each side of every line of its rule (16, 32, 64 and
     128 rows) gives the bits of the 64 x 64 tile."""
