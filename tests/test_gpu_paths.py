@@ -79,8 +79,8 @@ def test_attention_key_mask(be, T, W, hw_exp):
                                       (65, 640, 1024, None), (4111, 72, 640, 8)])
 def test_matmul_int4_chunked(be, T, N, K, zp, x_f32):
     """The K % 128 == 0 kernel: partial token and column tiles, odd, even and
-    compile-time chunk counts, zero-points of every block, both activation
-    forms and the 64-token tile. The f32 output against the oracle: both sum the
+    compile-time chunk counts, zero-points of every block and both activation
+    forms. The f32 output against the oracle: both sum the
     same per-block products in f32, so the difference is a few f32 ulps of the
     largest partial sum (K / 32 blocks: 2^-23 sqrt(K / 32) relative, times 4), plus 2^-22 for the hi/lo split."""
     w = synth.qweight(1300 + K, N, K, zp=zp)
@@ -94,24 +94,57 @@ def test_matmul_int4_chunked(be, T, N, K, zp, x_f32):
     assert err < 4 * 2.0 ** -23 * np.sqrt(K / 32) + 2.0 ** -22
 
 
-def test_matmul_int4_grid_limit():
-    """A product whose 32 x 64 tiles would be 2^24 workgroups of 256 threads
-    (a launch holds fewer than 2^32 threads) runs on the larger tiles: 64 GiB
-    of output, checked at the first, middle and last rows against a small call."""
-    T, N, K, n = (1 << 24) - 1, 2052, 128, 40
+@pytest.mark.parametrize("x_f32", [True, False], ids=["f32", "fp16"])
+@pytest.mark.parametrize("T,N,K", [(2432, 640, 896), (2433, 640, 896), (2496, 1152, 640), (2497, 1150, 640),
+                                   (2497, 1152, 384), (22465, 97, 128), (22465, 160, 128)])
+def test_matmul_int4_tile_rule(be, T, N, K, x_f32):
+    """Each side of the lines of the dense tile rule on 256 CUs (64 x 64 for fp16 input
+    from 2433 x 640, 64 x 128 for f32 from 2497 x 1152 and 22465 x 97, not where 160
+    columns would be padded to 256), with partial tiles, even and odd chunk counts: the bits of
+    the small tiles, which calls of at most 700 rows take."""
+    w = synth.qweight(1320 + K, N, K)
+    wb = [be.buffer(w[k]) for k in ("int4", "scales", "zp", "bias")]
+    x = synth.normal(1321, T * K).astype(np.float32).reshape(T, K)
+    x = x if x_f32 else synth.to_fp16_bits(x).reshape(T, K)
+    for o, dt in (("f16", np.uint16), ("f32", np.uint32)):
+        name = ("matmul_int4_f32_" if x_f32 else "matmul_int4_fp16_") + o
+        got = []
+        for rows in (T, 700):
+            for i in range(0, T, rows):
+                xb = be.buffer(np.ascontiguousarray(x[i:i + rows]))
+                n = min(rows, T - i)
+                out = be.buffer(nbytes=n * N * dt().nbytes)
+                be.dispatch(name, [xb] + wb + [out], u32s(n, N, K, 0))
+                got.append(out.read(dt).reshape(n, N))
+                xb.release()
+                out.release()
+        assert np.array_equal(got[0], np.concatenate(got[1:])), name
+    for b in wb:
+        b.release()
+
+
+@pytest.mark.parametrize("x_f32,N", [(True, 2052), (False, 4100)], ids=["f32", "fp16"])
+def test_matmul_int4_grid_limit(x_f32, N):
+    """Products whose small tiles (32 x 64 for 2052 columns, 64 x 64 for 4100) would be 2^24
+    workgroups of 256 threads or more (a launch holds fewer than 2^32 threads) run on
+    larger ones: 64 and 128 GiB of output, checked at the first, middle and last rows
+    against a small call."""
+    T, K, n = (1 << 24) - 1, 128, 40
     w = synth.qweight(1350, N, K)
     x = synth.normal(1351, 3 * n * K).astype(np.float32).reshape(3, n, K)
+    x, name = (x, "matmul_int4_f32_f16") if x_f32 else (synth.to_fp16_bits(x).reshape(3, n, K), "matmul_int4_fp16_f16")
+    row = x[0, 0].nbytes
     be = _native.Backend(0)  # its own: the scratch planes (8 GiB) go with it
     try:
         wb = [be.buffer(w[k]) for k in ("int4", "scales", "zp", "bias")]
-        xb, out = be.buffer(nbytes=T * K * 4), be.buffer(nbytes=T * N * 2)
-        be.dispatch("zero_f32", [xb], u32s(T * K, 0, 0, 0))
+        xb, out = be.buffer(nbytes=T * row), be.buffer(nbytes=T * N * 2)
+        be.dispatch("zero_f32", [xb], u32s(T * row // 4, 0, 0, 0))
         at = [0, T // 2, T - n]
         for r, v in zip(at, x):
-            xb.write(v, r * K * 4)
-        be.dispatch("matmul_int4_f32_f16", [xb] + wb + [out], u32s(T, N, K, 0))
+            xb.write(v, r * row)
+        be.dispatch(name, [xb] + wb + [out], u32s(T, N, K, 0))
         for r, v in zip(at, x):
-            ref = run(be, "matmul_int4_f32_f16", [v] + [w[k] for k in ("int4", "scales", "zp", "bias")], n * N * 2,
+            ref = run(be, name, [v] + [w[k] for k in ("int4", "scales", "zp", "bias")], n * N * 2,
                       u32s(n, N, K, 0)).view(np.uint16)
             assert np.array_equal(out.read(np.uint16, n * N, r * N * 2), ref), r
         for b in wb + [xb, out]:

@@ -615,10 +615,20 @@ bool launch_k128(pfhip_backend* b, const GemmArgs& a, const char* name) {
 
 // The tiles below, for the forms that the split forward and the named
 // products use; false: not built, or too many workgroups (the kernel above takes them).
-// Dense: 32 tokens x 64 columns at every size (2048 x 1152 x 640, RoPE
-// epilogue: 21.7 us, against 24.4 with 64 x 64 and 34.7 with 64 x 128), but 64
-// tokens from 4096 rows for one fp16 plane (O projection of 8192 rows: 24.3
-// against 28.9 us).
+// Dense: 32 tokens x 64 columns while the tiles are few. From 1.5 64 x 64 tiles per
+// CU on, 64 x 64 for one fp16 plane; from 1.375 64 x 128 tiles per CU on, 64 x 128
+// for split planes, unless 128 columns pad N by over an eighth more than 64 do. A tile of
+// twice the size dequantises (64 tokens) and reads activations (128 columns) half as
+// often, which counts once the CUs have several tiles to run; the line by rows (4096,
+// fp16 only) before this one left 9000 x 8192 x 512 behind the kernel above.
+// us on the kernel above / 32 x 64 / 64 x 64 / 64 x 128 (host call, 20 us more than
+// the kernel; split with the f32 -> hi + lo pass):
+//   fp16   1000 x 1152 x 640  52.4 / 30.2 / 30.4 / 33.1     1400 x 1152 x 640  52.4 / 32.9 / 31.2 / 33.4
+//          4095 x 4096 x 1024  169.7 / 174.1 / 141.2 / 139.9   20000 x 1152 x 640  168.8 / 153.8 / 126.9 / 134.7
+//   split  2048 x 1152 x 640  91.8 / 62.2 / 66.2 / 65.7     3000 x 1152 x 640  96.2 / 73.0 / 75.2 / 71.2
+//          9000 x 8192 x 512  529.8 / 542.6 / 546.0 / 441.2   20000 x 1152 x 640  265.9 / 249.6 / 250.8 / 211.1
+// With the RoPE epilogue 32 x 64 at every size (2048 x 1152 x 640: 21.7 us, against 24.4 with
+// 64 x 64 and 34.7 with 64 x 128; 32768 rows: 207, 232 and 207).
 // Grouped: the expert plan's tile. 16 and 32 rows take 64 columns, 64 rows 128 (gate_up
 // over 13.6 rows per expert: 26.6 / 30.0 / 41.0 us on tiles of 16 / 32 / 64
 // rows; over 64: 75.7 / 66.3 / 66.3; over 256: 281 / 227 / 197).
@@ -641,14 +651,20 @@ bool dispatch_k128(pfhip_backend* b, const GemmArgs& a, bool split, Epi epi, boo
     if (tile_t == 64) return tile(I2{}, std::integral_constant<int, 64>{});
     return false;
   }
+  const auto up = [](long n, long d) { return (n + d - 1) / d; };
+  const long rows64 = up(a.M, 64), cols64 = up(a.N, 64), cols128 = up(a.N, 128);
+  const bool large = split ? 8 * rows64 * cols128 >= 11L * b->num_cus && 16 * cols128 <= 9 * cols64
+                           : 2 * rows64 * cols64 >= 3L * b->num_cus;
   switch (epi) {
     case Epi::F16:
+      if (split && large) return launch_k128<2, 64, true, Epi::F16, false>(b, a, name);
       if (split) return launch_k128<1, 32, true, Epi::F16, false>(b, a, name);
-      if (a.M >= 4096) return launch_k128<1, 64, false, Epi::F16, false>(b, a, name);
+      if (large) return launch_k128<1, 64, false, Epi::F16, false>(b, a, name);
       return launch_k128<1, 32, false, Epi::F16, false>(b, a, name);
     case Epi::F32:
+      if (split && large) return launch_k128<2, 64, true, Epi::F32, false>(b, a, name);
       if (split) return launch_k128<1, 32, true, Epi::F32, false>(b, a, name);
-      if (a.M >= 4096) return launch_k128<1, 64, false, Epi::F32, false>(b, a, name);
+      if (large) return launch_k128<1, 64, false, Epi::F32, false>(b, a, name);
       return launch_k128<1, 32, false, Epi::F32, false>(b, a, name);
     case Epi::ROPE_F16:
       return split && launch_k128<1, 32, true, Epi::ROPE_F16, false>(b, a, name);
