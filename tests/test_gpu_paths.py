@@ -95,11 +95,11 @@ def test_matmul_int4_chunked(be, T, N, K, zp, x_f32):
 
 
 @pytest.mark.parametrize("x_f32", [True, False], ids=["f32", "fp16"])
-@pytest.mark.parametrize("T,N,K", [(2432, 640, 896), (2433, 640, 896), (2496, 1152, 640), (2497, 1150, 640),
-                                   (2497, 1152, 384), (22465, 97, 128), (22465, 160, 128)])
+@pytest.mark.parametrize("T,N,K", [(2432, 640, 896), (2433, 640, 896), (4544, 1152, 640), (4545, 1150, 640),
+                                   (4545, 1152, 384), (40897, 97, 128), (40897, 160, 128)])
 def test_matmul_int4_tile_rule(be, T, N, K, x_f32):
     """Each side of the lines of the dense tile rule on 256 CUs (64 x 64 for fp16 input
-    from 2433 x 640, 64 x 128 for f32 from 2497 x 1152 and 22465 x 97, not where 160
+    from 2433 x 640, 64 x 128 for f32 from 4545 x 1152 and 40897 x 97, not where 160
     columns would be padded to 256), with partial tiles, even and odd chunk counts: the bits of
     the small tiles, which calls of at most 700 rows take."""
     w = synth.qweight(1320 + K, N, K)

@@ -615,17 +615,19 @@ bool launch_k128(pfhip_backend* b, const GemmArgs& a, const char* name) {
 
 // The tiles below, for the forms that the split forward and the named
 // products use; false: not built, or too many workgroups (the kernel above takes them).
-// Dense: 32 tokens x 64 columns while the tiles are few. From 1.5 64 x 64 tiles per
-// CU on, 64 x 64 for one fp16 plane; from 1.375 64 x 128 tiles per CU on, 64 x 128
-// for split planes, unless 128 columns pad N by over an eighth more than 64 do. A tile of
+// Dense: 32 tokens x 64 columns while the tiles are few. Above 1.5 64 x 64 tiles per
+// CU, 64 x 64 for one fp16 plane; from 2.5 64 x 128 tiles per CU on, 64 x 128 for
+// split planes, unless 128 columns pad N by over an eighth more than 64 do. A tile of
 // twice the size dequantises (64 tokens) and reads activations (128 columns) half as
-// often, which counts once the CUs have several tiles to run; the line by rows (4096,
-// fp16 only) before this one left 9000 x 8192 x 512 behind the kernel above.
-// us on the kernel above / 32 x 64 / 64 x 64 / 64 x 128 (host call, 20 us more than
-// the kernel; split with the f32 -> hi + lo pass):
-//   fp16   1000 x 1152 x 640  52.4 / 30.2 / 30.4 / 33.1     1400 x 1152 x 640  52.4 / 32.9 / 31.2 / 33.4
+// often, which counts once every CU has several to run; the line by rows (4096,
+// fp16 only) before this one left 9000 x 8192 x 512 behind the kernel above. Over 938
+// products every choice is ahead of the kernel above; the larger tile is up to 3 % behind 32 x 64
+// for split planes and 5 % for one (1602 x 1280 x 640, just above two rounds).
+// us on the kernel above / 32 x 64 / 64 x 64 / 64 x 128 (events around the call: 15 to 20 us
+// more than the kernel; split with the f32 -> hi + lo pass):
+//   fp16   1290 x 1152 x 640  52.1 / 30.4 / 30.8 / -        1400 x 1152 x 640  52.4 / 32.9 / 31.2 / 33.4
 //          4095 x 4096 x 1024  169.7 / 174.1 / 141.2 / 139.9   20000 x 1152 x 640  168.8 / 153.8 / 126.9 / 134.7
-//   split  2048 x 1152 x 640  91.8 / 62.2 / 66.2 / 65.7     3000 x 1152 x 640  96.2 / 73.0 / 75.2 / 71.2
+//   split  3622 x 1152 x 640  110.6 / 80.7 / - / 83.1       4908 x 1152 x 640  122.5 / 97.1 / - / 92.6
 //          9000 x 8192 x 512  529.8 / 542.6 / 546.0 / 441.2   20000 x 1152 x 640  265.9 / 249.6 / 250.8 / 211.1
 // With the RoPE epilogue 32 x 64 at every size (2048 x 1152 x 640: 21.7 us, against 24.4 with
 // 64 x 64 and 34.7 with 64 x 128; 32768 rows: 207, 232 and 207).
@@ -653,8 +655,8 @@ bool dispatch_k128(pfhip_backend* b, const GemmArgs& a, bool split, Epi epi, boo
   }
   const auto up = [](long n, long d) { return (n + d - 1) / d; };
   const long rows64 = up(a.M, 64), cols64 = up(a.N, 64), cols128 = up(a.N, 128);
-  const bool large = split ? 8 * rows64 * cols128 >= 11L * b->num_cus && 16 * cols128 <= 9 * cols64
-                           : 2 * rows64 * cols64 >= 3L * b->num_cus;
+  const bool large = split ? 2 * rows64 * cols128 >= 5L * b->num_cus && 16 * cols128 <= 9 * cols64
+                           : 2 * rows64 * cols64 > 3L * b->num_cus;
   switch (epi) {
     case Epi::F16:
       if (split && large) return launch_k128<2, 64, true, Epi::F16, false>(b, a, name);
